@@ -718,8 +718,9 @@ uint64_t supportMask(const GOp& g) {
 
 // g applied to a vector of 2^nq amplitudes whose bit b is global qubit q[b]
 // (every qubit of g is one of them), in FP64, with the same semantics as
-// the single-gate kernels
-void applySmall(const GOp& g, const int* q, int nq, std::complex<double>* v) {
+// the single-gate kernels; false, with v untouched, for a kind whose action is
+// not known on the host (a DENSEN matrix is in device memory)
+bool applySmall(const GOp& g, const int* q, int nq, std::complex<double>* v) {
     typedef std::complex<double> cx;
     auto loc = [&](uint64_t m) {
         uint32_t r = 0;
@@ -830,13 +831,31 @@ void applySmall(const GOp& g, const int* q, int nq, std::complex<double>* v) {
                 if (((j & k1) != 0) != ((j & k2) != 0)) v[j] *= g.f[0];
             break;
         }
-        default: break;
+        case F_DEPOL2: {
+            const uint32_t a = 1u << bitOf(g.targs[0]), b = 1u << bitOf(g.targs[1]);
+            const uint32_t braA = 1u << bitOf(g.targs[2]), braB = 1u << bitOf(g.targs[3]);
+            const uint32_t dA = a | braA, dB = b | braB;
+            for (int j = 0; j < D; j++) {
+                if (j & (dA | dB)) continue;
+                const cx share = g.f[1] * (v[j] + v[j | dA] + v[j | dB] + v[j | dA | dB]);
+                for (uint32_t w = 0; w < 16; w++) {
+                    const bool ka = w & 1, kb = w & 2, ba = w & 4, bb = w & 8;
+                    cx& x = v[j | (ka ? a : 0) | (kb ? b : 0) | (ba ? braA : 0) | (bb ? braB : 0)];
+                    x = ka == ba && kb == bb ? g.f[0] * x + share : g.f[2] * x;
+                }
+            }
+            break;
+        }
+        default: return false;
     }
+    return true;
 }
 
 // the BLOCK op of ops[from, to), whose qubits all lie in the BQ local
-// qubits of S; its matrix is appended to `blocks` as the MFMA operands
-TOp makeBlock(const GOp* ops, size_t from, size_t to, uint64_t S, const Layout& L, std::vector<float>& blocks) {
+// qubits of S; its matrix is appended to `blocks` as the MFMA operands.  False
+// if the matrix of some op is not known here (see applySmall).
+bool makeBlock(const GOp* ops, size_t from, size_t to, uint64_t S, const Layout& L, std::vector<float>& blocks,
+               TOp& t) {
     typedef std::complex<double> cx;
     const int D = 1 << BQ;
     int q[BQ];
@@ -847,7 +866,8 @@ TOp makeBlock(const GOp* ops, size_t from, size_t to, uint64_t S, const Layout& 
     for (int c = 0; c < D; c++) {
         cx v[D];
         for (int j = 0; j < D; j++) v[j] = (j == c) ? 1.0 : 0.0;
-        for (size_t i = from; i < to; i++) applySmall(ops[i], q, BQ, v);
+        for (size_t i = from; i < to; i++)
+            if (!applySmall(ops[i], q, BQ, v)) return false;
         for (int r = 0; r < D; r++) U[r * D + c] = v[r];
     }
     // A[r][kk] of the real form [[Re U, -Im U], [Im U, Re U]], packed as
@@ -865,13 +885,12 @@ TOp makeBlock(const GOp* ops, size_t from, size_t to, uint64_t S, const Layout& 
                 else val = kk < 32 ? u.imag() : u.real();
                 P[(2 * s + half) * 64 + lane] = (float)val;
             }
-    TOp t;
     std::memset(&t, 0, sizeof(t));
     t.h.kind = F_BLOCK;
     int* slots = reinterpret_cast<int*>(t.b);
     for (int b = 0; b < BQ; b++) slots[b] = L.slotOf[q[b]];
     t.b[3] = (uint64_t)off;
-    return t;
+    return true;
 }
 
 // ops whose action is confined to one or two qubits (controls included),
@@ -914,7 +933,7 @@ void fuse::mergePass(const GOp* ops, size_t num, uint64_t localMask, std::vector
         for (int c = 0; c < D; c++) {
             std::complex<double> v[8] = {};
             v[c] = 1.0;
-            for (uint32_t m : b.members) applySmall(ops[m], q, nq, v);
+            for (uint32_t m : b.members) (void)applySmall(ops[m], q, nq, v);  // knows every mergeable kind
             for (int r = 0; r < D; r++) M[r * D + c] = v[r];
         }
         GOp g;
@@ -1147,7 +1166,7 @@ void fuse::planPass(const GOp* ops, size_t num, int numQubits, uint64_t localMas
     a.numOps = (int)(prog.size() - start);
 }
 
-void fuse::planPassBlocks(const GOp* ops, size_t num, int numQubits, uint64_t localMask, int lowQubits,
+bool fuse::planPassBlocks(const GOp* ops, size_t num, int numQubits, uint64_t localMask, int lowQubits,
                           int blockMinGates, TileArgs& a, std::vector<TOp>& prog, std::vector<float>& blocks) {
     Layout L;
     passShape(numQubits, localMask, a, L);
@@ -1160,10 +1179,11 @@ void fuse::planPassBlocks(const GOp* ops, size_t num, int numQubits, uint64_t lo
     size_t pending = 0;  // first op not yet emitted
     size_t i = 0;
     while (i < num) {
-        // the longest run from i whose qubits fit BQ local qubits
+        // the longest run from i whose qubits fit BQ local qubits; the matrix
+        // of a DENSEN op is in device memory, so it is in no block
         uint64_t S = 0;
         size_t j = i;
-        for (; j < num; j++) {
+        for (; j < num && ops[j].kind != F_DENSEN; j++) {
             const uint64_t sup = supportMask(ops[j]);
             if (sup & ~localMask) break;
             const uint64_t u = S | sup;
@@ -1181,7 +1201,9 @@ void fuse::planPassBlocks(const GOp* ops, size_t num, int numQubits, uint64_t lo
             for (int qq = 0; qq < numQubits && __builtin_popcountll(S) < BQ; qq++)
                 if ((localMask >> qq) & 1ull) S |= 1ull << qq;
             if (!any) firstItemGroup = false;
-            prog.push_back(makeBlock(ops, i, j, S, L, blocks));
+            TOp block;
+            if (!makeBlock(ops, i, j, S, L, blocks, block)) return false;
+            prog.push_back(block);
             any = true;
             lastItemGroup = false;
             i = pending = j;
@@ -1204,6 +1226,7 @@ void fuse::planPassBlocks(const GOp* ops, size_t num, int numQubits, uint64_t lo
     a.lastDirect = lastItemGroup && (st.lastG & lowSlots) == 0;
     a.usesLds = true;
     a.numOps = (int)(prog.size() - start);
+    return true;
 }
 
 namespace fuse {
@@ -1450,8 +1473,11 @@ int launchPass(void* amps, const Queue& qu, const std::vector<GOp>& ops, size_t 
     prog.clear();
     if (qu.prec == QA_FP32 && g_cfg.blockMinGates > 0) {
         g_blockData.clear();
-        planPassBlocks(ops.data() + begin, end - begin, qu.numQubits, localMask, g_cfg.lowQubits, g_cfg.blockMinGates,
-                       a, prog, g_blockData);
+        if (!planPassBlocks(ops.data() + begin, end - begin, qu.numQubits, localMask, g_cfg.lowQubits,
+                            g_cfg.blockMinGates, a, prog, g_blockData)) {
+            setError("fusion: an MFMA block cannot hold one of its gates");
+            return QA_ERR_ARG;
+        }
         if (!g_blockData.empty()) {
             const size_t nf = g_blockData.size();
             if (nf > BLOCK_RING_FLOATS) {

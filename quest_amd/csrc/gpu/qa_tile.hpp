@@ -123,8 +123,9 @@ struct LayerFrame {
 // the same for a complex64 state, where runs of at least blockMinGates ops
 // whose qubits (targets, controls, masks) fit 5 local qubits become one
 // BLOCK op; their packed 32x32 matrices are appended to `blocks` and each
-// BLOCK op holds its offset there (a.blocks is left for the caller)
-void planPassBlocks(const GOp* ops, size_t num, int numQubits, uint64_t localMask, int lowQubits, int blockMinGates,
+// BLOCK op holds its offset there (a.blocks is left for the caller).  False
+// when a block would hold an op whose action the host does not know.
+bool planPassBlocks(const GOp* ops, size_t num, int numQubits, uint64_t localMask, int lowQubits, int blockMinGates,
                     TileArgs& a, std::vector<TOp>& prog, std::vector<float>& blocks);
 
 // the LDS byte offsets of the register layouts of a planned pass (prog[0..num),

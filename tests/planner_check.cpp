@@ -148,6 +148,22 @@ static void apply(const GOp& g, std::vector<cx>& a) {
                 if (((i & k1) != 0) != ((i & k2) != 0)) a[i] *= g.f[0];
             break;
         }
+        case F_DEPOL2: {
+            // every amplitude scales; the 4 of a group with ket = bra on both
+            // qubits then share a multiple of their sum
+            const uint64_t k1 = 1ull << g.targs[0], k2 = 1ull << g.targs[1], b1 = 1ull << g.targs[2], b2 = 1ull << g.targs[3];
+            for (uint64_t i = 0; i < N; i++) {
+                if (i & (k1 | k2 | b1 | b2)) continue;
+                cx sum = 0;
+                for (int v = 0; v < 4; v++) sum += a[i | (v & 1 ? k1 | b1 : 0) | (v & 2 ? k2 | b2 : 0)];
+                for (int v = 0; v < 16; v++) {
+                    const uint64_t j = i | (v & 1 ? k1 : 0) | (v & 2 ? k2 : 0) | (v & 4 ? b1 : 0) | (v & 8 ? b2 : 0);
+                    if ((v & 3) == (v >> 2)) a[j] = g.f[0] * a[j] + g.f[1] * sum;
+                    else a[j] *= g.f[2];
+                }
+            }
+            break;
+        }
         default:
             std::fprintf(stderr, "unknown op kind %d\n", g.kind);
             std::exit(3);
@@ -210,6 +226,20 @@ static GOp randomGate(Rng& r, int n, bool dens, int hot) {
         for (double& x : pool.back()) x = r.unit() / D;
         g.mat = pool.back().data();
         g.conj = r.below(2);
+        return g;
+    }
+    if (dens && n >= 4 && r.below(12) == 0) {
+        // two-qubit depolarising, weak or as strong as it gets
+        g.kind = F_DEPOL2;
+        g.numTargs = 4;
+        g.targs[0] = r.below(n / 2);
+        do g.targs[1] = r.below(n / 2); while (g.targs[1] == g.targs[0]);
+        g.targs[2] = g.targs[0] + n / 2;
+        g.targs[3] = g.targs[1] + n / 2;
+        const double p = r.below(2) ? 15.0 / 16 : 0.05 * (r.unit() + 1);
+        g.f[0] = 1 - 16 * p / 15;
+        g.f[1] = 4 * p / 15;
+        g.f[2] = 1 - 16 * p / 15;
         return g;
     }
     const int kind = r.below(dens ? 10 : 8);
@@ -649,9 +679,106 @@ static int spanMain(int cases, uint64_t seed0) {
     return 0;
 }
 
+// ---- MFMA blocks ------------------------------------------------------------
+
+// random passes of gates on a few qubits planned with blocks from one gate on,
+// so that a program is BLOCK ops and, between them, the 3- and 4-qubit
+// matrices that stay on the device; the BLOCK matrices, unpacked, and those
+// matrices applied to a state must act like the gates, to the rounding of the
+// packed FP32 elements
+static int blocksMain(int cases, uint64_t seed0) {
+    int numBlocks = 0, numLds = 0, numDepol = 0;
+    for (int c = 0; c < cases; c++) {
+        Rng r(seed0 * 104729ull + (uint64_t)c);
+        const bool dens = c % 2;
+        const int n = dens ? 10 : 10 + r.below(3), k = n;
+        std::vector<GOp> queue;
+        for (int i = 2 + r.below(12); i > 0; i--) {
+            GOp g = randomGate(r, n, dens, 4);
+            if (__builtin_popcountll(supportMask(g)) > BQ) continue;
+            numDepol += g.kind == F_DEPOL2;
+            queue.push_back(g);
+        }
+        std::vector<cx> want(1ull << n);
+        for (auto& x : want) x = cx(r.unit(), r.unit());
+        std::vector<cx> got = want;
+        for (const GOp& g : queue) ::apply(g, want);
+        TileArgs a;
+        std::vector<TOp> prog;
+        std::vector<float> blocks;
+        planPassBlocks(queue.data(), queue.size(), n, (1ull << k) - 1ull, r.below(4), 1, a, prog, blocks);
+        for (const TOp& t : prog) {
+            const int* w = reinterpret_cast<const int*>(t.b);
+            if (t.h.kind == F_GROUP) continue;
+            GOp g;
+            std::vector<double> mat;
+            if (t.h.kind == F_DENSE_LDS) {
+                numLds++;
+                g.numTargs = w[4];
+                g.conj = w[5];
+                g.mat = reinterpret_cast<const double*>((uintptr_t)(uint32_t)w[6] | (uintptr_t)(uint32_t)w[7] << 32);
+            } else if (t.h.kind == F_BLOCK) {
+                numBlocks++;
+                const float* P = blocks.data() + t.b[3];
+                const int D = 1 << BQ;
+                // element (row, column) of the real form's left half: Re U over Im U
+                auto at = [&](int half, int row, int col) {
+                    return (double)P[(2 * (col / 2) + half) * 64 + row + 32 * (col % 2)];
+                };
+                for (int row = 0; row < D; row++)
+                    for (int col = 0; col < D; col++) {
+                        mat.push_back(at(0, row, col));
+                        mat.push_back(at(1, row, col));
+                    }
+                g.numTargs = BQ;
+                g.mat = mat.data();
+            } else {
+                std::printf("case %d: op kind %d in a pass of blocks\n", c, t.h.kind);
+                return 1;
+            }
+            int q[BQ];
+            for (int b = 0; b < g.numTargs; b++) q[b] = a.localPos[w[b]];
+            const int D = 1 << g.numTargs;
+            uint64_t tm = 0;
+            for (int b = 0; b < g.numTargs; b++) tm |= 1ull << q[b];
+            for (uint64_t i = 0; i < got.size(); i++) {
+                if (i & tm) continue;
+                std::vector<cx> x(D);
+                std::vector<uint64_t> j(D, i);
+                for (int v = 0; v < D; v++) {
+                    for (int b = 0; b < g.numTargs; b++)
+                        if ((v >> b) & 1) j[v] |= 1ull << q[b];
+                    x[v] = got[j[v]];
+                }
+                for (int row = 0; row < D; row++) {
+                    cx y = 0;
+                    for (int col = 0; col < D; col++)
+                        y += cx(g.mat[2 * (row * D + col)], (g.conj ? -1 : 1) * g.mat[2 * (row * D + col) + 1]) * x[col];
+                    got[j[row]] = y;
+                }
+            }
+        }
+        // every block's elements are rounded to FP32 once
+        double err = 0, norm = 0;
+        for (size_t i = 0; i < got.size(); i++) {
+            err += std::norm(got[i] - want[i]);
+            norm += std::norm(want[i]);
+        }
+        if (!(std::sqrt(err) <= 1e-5 * std::sqrt(norm) + 1e-12)) {
+            std::printf("case %d (n=%d gates=%zu): error %.3e of %.3e\n", c, n, queue.size(), std::sqrt(err),
+                        std::sqrt(norm));
+            return 1;
+        }
+    }
+    std::printf("block check: %d cases agree (%d blocks, %d matrices, %d two-qubit depolarising)\n", cases, numBlocks,
+                numLds, numDepol);
+    return numBlocks && numLds && numDepol ? 0 : 1;
+}
+
 int main(int argc, char** argv) {
     const int cases = argc > 1 ? std::atoi(argv[1]) : 200;
     const uint64_t seed0 = argc > 2 ? std::strtoull(argv[2], nullptr, 10) : 1;
+    if (argc > 3 && std::string(argv[3]) == "blocks") return blocksMain(cases, seed0);
     if (argc > 3 && std::string(argv[3]) == "span") return spanMain(cases, seed0);
     JitCheck jit;
     if (argc > 3 && std::string(argv[3]) == "jit") {

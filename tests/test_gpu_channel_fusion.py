@@ -81,3 +81,36 @@ def test_channels_in_passes_match_their_own_kernels(api):
         api.set_fusion(bool(before[0]), *before[1:])
     assert rel(amps[0], amps[1]) <= 1e-13
     assert np.array_equal(amps[1], amps[2])  # exact fusion keeps the channels' own kernels
+
+
+@pytest.mark.parametrize("min_gates", [1, 2])
+def test_channels_in_mfma_blocks(api, min_gates):
+    """complex64 passes whose runs on 5 index bits are multiplied into one
+    32x32 matrix hold the channels too, strong ones so that a lost one shows;
+    3-target matrices end a run.  A gate rounds the state by at most a few
+    2^-24, and a block's elements are rounded once."""
+    from oracle import qoracle as O
+    print(f"[gpu] channels in MFMA blocks, from {min_gates} gates", flush=True)
+    before = api.get_fusion()
+    n = 6
+    rng = qc.SplitMix64(61)
+    c = qc.Circuit(n, True, [], ("random", 62), "channels_blocks")
+    for i in range(24):
+        a, b = rng.sample(n, 2)
+        c.ops.append([("DEPOL2", a, b, 0.5), ("DEPH2", a, b, 0.4), ("DAMP", a, 0.3), ("PAULIS", b, 0.1, 0.2, 0.05)][i % 4])
+        if i % 3 == 0:
+            c.ops.append(("U1", a, qc.haar_unitary(rng, 2)))
+        if i % 8 == 5:
+            c.ops.append(("UN", rng.sample(n, 3), qc.haar_unitary(rng, 8)))
+    want, _ = O.run(c)
+    api.set_fusion(True, 10, 3, 512)
+    assert api.gpu().qa_setFusionBlocks(min_gates) == 0
+    try:
+        q = api.createCustomPrecisionQureg(n, 1, 1)
+        q, _ = qc.run(c, q)
+        got = api.get_amps(q)
+        api.destroyQureg(q)
+    finally:
+        api.gpu().qa_setFusionBlocks(0)
+        api.set_fusion(bool(before[0]), *before[1:])
+    assert rel(got, want) <= 8 * 2.0 ** -24 * len(c.ops)

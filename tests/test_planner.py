@@ -50,6 +50,16 @@ def test_span_passes_act_like_the_gadgets(planner_check, seed):
     assert "300 cases agree" in out.stdout
 
 
+@pytest.mark.parametrize("seed", [1, 2])
+def test_blocks_act_like_their_gates(planner_check, seed):
+    """MFMA blocks of complex64 passes: every kind of gate whose qubits fit a
+    block, two-qubit depolarising among them, is in the block's matrix, and 3-
+    and 4-qubit matrices, whose elements are on the device, end a block."""
+    out = subprocess.run([str(planner_check), "200", str(seed), "blocks"], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, out.stdout + out.stderr
+    assert "200 cases agree" in out.stdout
+
+
 def test_generated_pass_kernels_compile_and_cache_soundly(planner_check):
     """Every planned pass program also gets its generated kernel source:
     programs with equal shape keys must generate equal sources (the per-shape
