@@ -446,25 +446,33 @@ SignTerm signTerm(const GOp& g, const Layout& L) {
     return t;
 }
 
-// g as phase * scale * diag(1, after) [[1, -t], [t, 1]] diag(1, before), the
-// phase and scale in `factor`; false when it is not unitary or its diagonal is
-// so small that the scaled amplitudes would leave the storage's middle range
-bool splitUnitary(const double* m, std::complex<double>& factor, std::complex<double>& before,
+// m as factor * diag(1, after) [[1, -t], [t, 1]] diag(1, before), `factor`
+// being its first element and the phases of modulus 1; false (a DENSE1 op is
+// then made of it) when it is not unitary, or when its diagonal is so small
+// that the scaled amplitudes would leave the storage's middle range.  The
+// element b is not used but follows from the others, so "unitary" is to a few
+// units of FP64 in a complex128 state (rotations, their products and Haar
+// matrices are within 1 to 3 of 2^-52) and well below a unit of the storage in
+// a complex64 one; a NaN in any element fails the comparisons.
+bool splitUnitary(const double* m, int prec, std::complex<double>& factor, std::complex<double>& before,
                   std::complex<double>& after, double& t) {
     typedef std::complex<double> cx;
     const cx a(m[0], m[1]), b(m[2], m[3]), c(m[4], m[5]), d(m[6], m[7]);
-    const double eps = 1e-13;
-    if (std::abs(std::norm(a) + std::norm(c) - 1) > eps || std::abs(std::norm(b) + std::norm(d) - 1) > eps ||
-        std::abs(std::conj(a) * b + std::conj(c) * d) > eps)
+    const double eps = prec == QA_FP64 ? 0x1p-50 : 1e-13;
+    if (!(std::abs(std::norm(a) + std::norm(c) - 1) <= eps && std::abs(std::norm(b) + std::norm(d) - 1) <= eps &&
+          std::abs(std::conj(a) * b + std::conj(c) * d) <= eps))
         return false;
-    const double co = std::abs(a), si = std::abs(c);
+    const double co = std::abs(a);
     if (co < 1.0 / 256) return false;
     const cx e = a / co;
     factor = a;
-    t = si / co;
+    t = std::abs(c) / co;
     // `after` from c and `before` from d, so that an error of after's phase
-    // (c may be small) is not in d; b follows from the others
-    after = si > 0 ? c / (e * si) : cx(1);
+    // (c may be small) is not in d.  A c among the subnormals has few bits, and
+    // a quotient of two of them fewer: its phase is taken from c scaled up.
+    const cx up = std::norm(c) < 0x1p-900 ? c * 0x1p+900 : c;
+    after = up == cx(0) ? cx(1) : up / (e * std::abs(up));
+    after /= std::abs(after);
     before = d / (e * after);
     before /= std::abs(before);
     return true;
@@ -506,7 +514,7 @@ size_t layerOp(const GOp* ops, size_t num, const Layout& L, LayerFrame& frame, s
         const int q = ops[n].t1, b = L.regOf[L.slotOf[q]];
         if ((mask >> b) & 1) break;
         cx factor;
-        if (!splitUnitary(ops[n].f, factor, before[b], after[b], rot[b])) break;
+        if (!splitUnitary(ops[n].f, frame.prec, factor, before[b], after[b], rot[b])) break;
         scale *= factor;
         before[b] *= frame.f[q];
         qubit[b] = q;

@@ -27,7 +27,97 @@ static void dense1(std::vector<cx>& v, int q, const double* m) {
     }
 }
 
+// One matrix, planned with a frame on a state of its own: the program must
+// apply the matrix that was given, to a few ulp of FP64, whether or not it is
+// exactly unitary.
+static bool oneMatrix(const cx (&m)[4], const char* what) {
+    const int n = 4;
+    GOp g;
+    g.kind = F_DENSE1;
+    g.t1 = 2;
+    for (int k = 0; k < 4; k++) g.f[2 * k] = m[k].real(), g.f[2 * k + 1] = m[k].imag();
+    LayerFrame frame;
+    frame.finish = true;
+    TileArgs a;
+    std::vector<TOp> prog;
+    planPass(&g, 1, n, (1ull << n) - 1, 0, a, prog, true, true, &frame);
+    // each column of the product of the program's ops on the one qubit
+    double worst = 0;
+    for (int col = 0; col < 2; col++) {
+        cx v[2] = {col == 0 ? 1.0 : 0.0, col == 1 ? 1.0 : 0.0};
+        int reg = -1;  // the qubit's register bit
+        for (const TOp& t : prog) {
+            const double* b = reinterpret_cast<const double*>(t.b);
+            if (t.h.kind == F_GROUP) {
+                for (int r = 0; r < RB; r++)
+                    if (a.localPos[reinterpret_cast<const int*>(t.b)[r]] == g.t1) reg = r;
+            } else if (t.h.kind == F_DENSE1) {
+                const cx x = v[0], y = v[1];
+                v[0] = at(b, 0) * x + at(b, 1) * y;
+                v[1] = at(b, 2) * x + at(b, 3) * y;
+            } else if (t.h.kind == F_DIAG1) {
+                v[1] *= at(b, 1);
+                if (!t.h.pad) v[0] *= at(b, 0);
+            } else if (t.h.kind == F_LAYER) {
+                const LayerBody<double>& body = *reinterpret_cast<const LayerBody<double>*>(t.b);
+                for (int r = 0; r < 2; r++) {
+                    const int w = r << reg;
+                    v[r] *= cx(body.factor[2 * w], body.factor[2 * w + 1]);
+                }
+                const cx x = v[0], y = v[1];
+                v[0] = x - body.t[reg] * y;
+                v[1] = body.t[reg] * x + y;
+            } else {
+                std::printf("FAIL: %s: op kind %d\n", what, t.h.kind);
+                return false;
+            }
+        }
+        for (int r = 0; r < 2; r++) {
+            const double off = std::abs(v[r] - m[2 * r + col]);
+            worst = std::isnan(off) ? INFINITY : std::max(worst, off);
+        }
+    }
+    if (worst <= 8 * 2.3e-16) return true;
+    std::printf("FAIL: %s: an element is off by %.3e\n", what, worst);
+    return false;
+}
+
+static bool matrices() {
+    const double h = std::sqrt(0.5), nan = std::nan("");
+    const cx e = std::polar(1.0, 2.45), f = std::polar(1.0, -0.7);
+    for (double th : {5e-324, 2e-323, 1e-322, 1e-320, 1e-318, 1e-300, 1e-160, 0.3}) {
+        const double c = std::cos(th), s = std::sin(th);
+        // a rotation, then a phase
+        const cx m[4] = {c, -s, e * s, e * c};
+        if (!oneMatrix(m, "small angle")) return false;
+    }
+    for (double d : {4e-14, 1e-14, 3e-15}) {
+        const cx b[4] = {0.6 * f, -0.8 * (1 + d), 0.8 * f * e, 0.6 * e}, a[4] = {h, h, h, -h * (1 - d)};
+        if (!oneMatrix(b, "nearly unitary") || !oneMatrix(a, "nearly unitary")) return false;
+    }
+    for (int k = 0; k < 4; k++) {
+        cx m[4] = {h, h, h, -h};
+        m[k] = cx(nan, 0);
+        LayerFrame frame;
+        frame.finish = true;
+        GOp g;
+        g.kind = F_DENSE1;
+        g.t1 = 2;
+        for (int i = 0; i < 4; i++) g.f[2 * i] = m[i].real(), g.f[2 * i + 1] = m[i].imag();
+        TileArgs a;
+        std::vector<TOp> prog;
+        planPass(&g, 1, 4, 15, 0, a, prog, true, true, &frame);
+        // a matrix that is no unitary goes as it is
+        bool kept = false;
+        for (const TOp& t : prog)
+            if (t.h.kind == F_DENSE1) kept = std::isnan(reinterpret_cast<const double*>(t.b)[2 * k]);
+        if (!kept) return std::printf("FAIL: a NaN element of a matrix is lost\n"), false;
+    }
+    return true;
+}
+
 int main(int argc, char** argv) {
+    if (!matrices()) return 1;
     const int rounds = argc > 1 ? std::atoi(argv[1]) : 200;
     std::mt19937_64 rng(argc > 2 ? std::strtoull(argv[2], nullptr, 0) : 1);
     auto below = [&](int n) { return (int)(rng() % (uint64_t)n); };
@@ -48,8 +138,9 @@ int main(int argc, char** argv) {
                 if (framed && below(8)) {
                     // e^{ia} [[c, -s e^{il}], [s e^{ip}, c e^{i(l+p)}]]: any angle, or a (nearly) diagonal or
                     // antidiagonal one
-                    const double special[] = {0, 1e-12, 1e-7, M_PI / 2, M_PI / 2 - 1e-5, M_PI, 0.78539816339744828};
-                    const double th = below(3) ? M_PI * uniform() : special[below(7)];
+                    const double special[] = {0, 1e-12, 1e-7, M_PI / 2, M_PI / 2 - 1e-5, M_PI, 0.78539816339744828,
+                                              5e-324, 2e-323, 1e-322, 1e-320, 1e-318, 1e-300, 1e-160, 1e-140};
+                    const double th = below(3) ? M_PI * uniform() : special[below(15)];
                     const double a = M_PI * uniform(), l = below(4) ? M_PI * uniform() : 0, p = below(4) ? M_PI * uniform() : 0;
                     const cx m[4] = {std::polar(1.0, a) * std::cos(th), -std::polar(1.0, a + l) * std::sin(th),
                                      std::polar(1.0, a + p) * std::sin(th), std::polar(1.0, a + l + p) * std::cos(th)};
