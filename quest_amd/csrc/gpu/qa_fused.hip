@@ -103,7 +103,8 @@ uint64_t denseMask(const GOp& g) {
             return m;
         }
         case F_DENSE1: case F_DENSE1V: return 1ull << g.t1;
-        case F_DENSE2: case F_SWAP: case F_DEPOL1: case F_DEPH1: return (1ull << g.t1) | (1ull << g.t2);
+        case F_DENSE2: case F_SWAP: case F_DEPOL1: case F_DEPH1: case F_DAMP1: case F_PAULIS1:
+            return (1ull << g.t1) | (1ull << g.t2);
         case F_PAULI: return g.m1;
         default: return 0;  // diagonal: any qubit
     }
@@ -184,7 +185,10 @@ TOp toTile(const GOp& g, const Layout& L) {
     auto regBit = [&](int q) { return (q >= 0 && L.slotOf[q] >= 0) ? L.regOf[L.slotOf[q]] : -1; };
     h.rb1 = regBit(g.t1);
     h.rb2 = regBit(g.t2);
-    if ((g.kind == F_SWAP || g.kind == F_DEPOL1 || g.kind == F_DEPH1) && h.rb1 > h.rb2) std::swap(h.rb1, h.rb2);
+    // kinds that act alike on (01) and (10)
+    if ((g.kind == F_SWAP || g.kind == F_DEPOL1 || g.kind == F_DEPH1 || g.kind == F_DAMP1 || g.kind == F_PAULIS1) &&
+        h.rb1 > h.rb2)
+        std::swap(h.rb1, h.rb2);
     uint32_t rv;
     uint64_t tv, gv;
     splitMask(g.cMask, L, h.rcMask, h.jcMask, h.gcMask);
@@ -839,6 +843,27 @@ bool applySmall(const GOp& g, const int* q, int nq, std::complex<double>* v) {
                 if (((j & k1) != 0) != ((j & k2) != 0)) v[j] *= g.f[0];
             break;
         }
+        case F_DAMP1: case F_PAULIS1: {
+            const uint32_t k1 = 1u << bitOf(g.t1), k2 = 1u << bitOf(g.t2);
+            const double* f = g.f;
+            for (int j = 0; j < D; j++) {
+                if (j & (k1 | k2)) continue;
+                cx &a00 = v[j], &a01 = v[j | k1], &a10 = v[j | k2], &a11 = v[j | k1 | k2];
+                if (g.kind == F_DAMP1) {
+                    a00 += f[0] * a11;
+                    a01 *= f[1];
+                    a10 *= f[1];
+                    a11 *= f[2];
+                } else {
+                    const cx x00 = a00, x01 = a01;
+                    a00 = f[0] * x00 + f[1] * a11;
+                    a11 = f[0] * a11 + f[1] * x00;
+                    a01 = f[2] * x01 + f[3] * a10;
+                    a10 = f[2] * a10 + f[3] * x01;
+                }
+            }
+            break;
+        }
         case F_DEPOL2: {
             const uint32_t a = 1u << bitOf(g.targs[0]), b = 1u << bitOf(g.targs[1]);
             const uint32_t braA = 1u << bitOf(g.targs[2]), braB = 1u << bitOf(g.targs[3]);
@@ -906,7 +931,7 @@ bool makeBlock(const GOp* ops, size_t from, size_t to, uint64_t S, const Layout&
 bool mergeable(const GOp& g) {
     switch (g.kind) {
         case F_DENSE1: case F_DENSE2: case F_DIAG1: case F_PARITY: case F_PAULI: case F_SWAP: case F_DEPOL1:
-        case F_DEPH1: break;
+        case F_DEPH1: case F_DAMP1: case F_PAULIS1: break;
         default: return false;
     }
     const int n = __builtin_popcountll(supportMask(g));
@@ -922,10 +947,19 @@ void fuse::mergePass(const GOp* ops, size_t num, uint64_t localMask, std::vector
         uint64_t variants;              // non-local qubits (members are diagonal in them)
         std::vector<uint32_t> members;  // positions in ops, ascending
         bool dense;                     // some member is not diagonal
+        bool matrix = false;            // some member is a matrix, or a Pauli tensor or gadget
+        bool channel = false;           // some member is a damping or Pauli channel
+        void note(const GOp& g) {
+            matrix |= g.kind == F_DENSE1 || g.kind == F_DENSE2 || g.kind == F_PAULI;
+            channel |= g.kind == F_DAMP1 || g.kind == F_PAULIS1;
+        }
     };
     std::vector<Block> open;  // pairwise disjoint qubit sets
     auto emit = [&](const Block& b) {
-        if (b.members.size() == 1 || !b.dense) {
+        // damping and Pauli channels that no matrix meets keep their own sums: as
+        // a 4x4 complex matrix they take more arithmetic, and its zeros turn
+        // an infinite amplitude into NaN all over its group
+        if (b.members.size() == 1 || !b.dense || (b.channel && !b.matrix)) {
             for (uint32_t m : b.members) out.push_back(ops[m]);
             return;
         }
@@ -998,6 +1032,8 @@ void fuse::mergePass(const GOp* ops, size_t num, uint64_t localMask, std::vector
             if (fits) {
                 nb.members.insert(nb.members.end(), open[b].members.begin(), open[b].members.end());
                 nb.dense |= open[b].dense;
+                nb.matrix |= open[b].matrix;
+                nb.channel |= open[b].channel;
             } else {
                 emit(open[b]);
             }
@@ -1009,6 +1045,7 @@ void fuse::mergePass(const GOp* ops, size_t num, uint64_t localMask, std::vector
         }
         std::sort(nb.members.begin(), nb.members.end());
         nb.members.push_back((uint32_t)i);
+        nb.note(g);
         open.push_back(std::move(nb));
     }
     for (const Block& b : open) emit(b);
@@ -1252,6 +1289,8 @@ double opFlops(const GOp& g, int n) {
         case F_PAULI: perAmp = 14; break;    // multiply + multiply-add per amplitude
         case F_DEPOL1: perAmp = 4; break;    // 16 per 4 amplitudes
         case F_DEPH1: perAmp = 1; break;     // 4 per 4 amplitudes
+        case F_DAMP1: perAmp = 2.5; break;   // 10 per 4 amplitudes
+        case F_PAULIS1: perAmp = 6; break;   // a multiply and a multiply-add each
         case F_DEPOL2: perAmp = 3; break;    // one multiply each, 4 of 16 also share a sum
         case F_DENSEN: perAmp = 8.0 * (1 << g.numTargs); break;  // 2^n complex MACs per amplitude
         default: perAmp = 0; break;

@@ -12,7 +12,7 @@ namespace fuse {
 // a queued gate in global index space
 struct GOp {
     int kind = 0;
-    int t1 = -1, t2 = -1;            // targets (DEPOL1/DEPH1: ket, bra)
+    int t1 = -1, t2 = -1;            // targets (one-qubit channels: ket, bra)
     uint64_t cMask = 0, cVal = 0;    // control condition: (i & cMask) == cVal
     uint64_t m1 = 0, m2 = 0;         // PARITY: parity mask; PAULI: maskXY, maskYZ; DENSE1V: variant qubits
     double f[32] = {0};              // matrix / factors (re, im interleaved); DENSE1V: one 2x2

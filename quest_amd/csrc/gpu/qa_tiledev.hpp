@@ -62,6 +62,7 @@ static_assert(sizeof(TOpHead) == 64, "op header is one 64-byte scalar load");
 //     parity mask (PARITY) or the maskYZ bits (PAULI) outside the
 //     registers, b[5] = its non-local part
 //   DEPOL1: b[0..2] = c1, c2, c3;  DEPH1: b[0] = factor
+//   DAMP1: b[0..2] = prob, c1, c2;  PAULIS1: b[0..3] = fAA, fBB, fAB, fBA
 //   DEPOL2: b[0..2] = c1 - c2, c2, 1 + c3; rb1 = the register bit that is the
 //     other half (bra or ket) of register bit 0's qubit
 //   GROUP: b[0..1] = the RB tile slots of the register bits (4 ints);
@@ -495,6 +496,36 @@ __device__ __forceinline__ void regDeph1(ct<T>* r, const double* f) {
     }
 }
 
+template <typename T, int B1, int B2>
+__device__ __forceinline__ void regDamp1(ct<T>* r, const double* f) {
+    const T prob = (T)f[0], c1 = (T)f[1], c2 = (T)f[2];
+#pragma unroll
+    for (int v = 0; v < RA; v++) {
+        if (v & ((1 << B1) | (1 << B2))) continue;
+        constexpr int k1 = 1 << B1, k2 = 1 << B2;
+        const ct<T> a00 = r[v], a01 = r[v | k1], a10 = r[v | k2], a11 = r[v | k1 | k2];
+        r[v] = ct<T>{fmaT(prob, a11.re, a00.re), fmaT(prob, a11.im, a00.im)};
+        r[v | k1] = ct<T>{c1 * a01.re, c1 * a01.im};
+        r[v | k2] = ct<T>{c1 * a10.re, c1 * a10.im};
+        r[v | k1 | k2] = ct<T>{c2 * a11.re, c2 * a11.im};
+    }
+}
+
+template <typename T, int B1, int B2>
+__device__ __forceinline__ void regPaulis1(ct<T>* r, const double* f) {
+    const T fAA = (T)f[0], fBB = (T)f[1], fAB = (T)f[2], fBA = (T)f[3];
+#pragma unroll
+    for (int v = 0; v < RA; v++) {
+        if (v & ((1 << B1) | (1 << B2))) continue;
+        constexpr int k1 = 1 << B1, k2 = 1 << B2;
+        const ct<T> a00 = r[v], a01 = r[v | k1], a10 = r[v | k2], a11 = r[v | k1 | k2];
+        r[v] = ct<T>{fmaT(fAA, a00.re, fBB * a11.re), fmaT(fAA, a00.im, fBB * a11.im)};
+        r[v | k1] = ct<T>{fmaT(fAB, a01.re, fBA * a10.re), fmaT(fAB, a01.im, fBA * a10.im)};
+        r[v | k2] = ct<T>{fmaT(fAB, a10.re, fBA * a01.re), fmaT(fAB, a10.im, fBA * a01.im)};
+        r[v | k1 | k2] = ct<T>{fmaT(fAA, a11.re, fBB * a00.re), fmaT(fAA, a11.im, fBB * a00.im)};
+    }
+}
+
 // two-qubit depolarising: the registers are the 16 amplitudes of one
 // (ket1, ket2, bra1, bra2) group, P the register bit paired (as ket and bra
 // of one qubit) with bit 0.  Every amplitude scales by f, and the 4 with ket
@@ -833,6 +864,16 @@ __device__ __forceinline__ void applyOp(ct<T>* r, const TOp* __restrict__ op, co
                 switch (h.rb1 * RB + h.rb2) { QA_CHAN_CASES(regDeph1) }
             }
             break;
+        case F_DAMP1:
+            if constexpr (!SV) {
+                switch (h.rb1 * RB + h.rb2) { QA_CHAN_CASES(regDamp1) }
+            }
+            break;
+        case F_PAULIS1:
+            if constexpr (!SV) {
+                switch (h.rb1 * RB + h.rb2) { QA_CHAN_CASES(regPaulis1) }
+            }
+            break;
         case F_DEPOL2:
             if constexpr (!SV) {
                 switch (h.rb1) {
@@ -907,6 +948,10 @@ __device__ __forceinline__ void applyFixed(ct<T>* r, const TOp* __restrict__ op,
         regDepol1<T, RB1, RB2>(r, f);
     } else if constexpr (KIND == F_DEPH1) {
         regDeph1<T, RB1, RB2>(r, f);
+    } else if constexpr (KIND == F_DAMP1) {
+        regDamp1<T, RB1, RB2>(r, f);
+    } else if constexpr (KIND == F_PAULIS1) {
+        regPaulis1<T, RB1, RB2>(r, f);
     } else if constexpr (KIND == F_DEPOL2) {
         regDepol2<T, RB1>(r, f);
     }

@@ -148,6 +148,25 @@ static void apply(const GOp& g, std::vector<cx>& a) {
                 if (((i & k1) != 0) != ((i & k2) != 0)) a[i] *= g.f[0];
             break;
         }
+        case F_DAMP1: case F_PAULIS1: {
+            const uint64_t k1 = 1ull << g.t1, k2 = 1ull << g.t2;
+            for (uint64_t i = 0; i < N; i++) {
+                if (i & (k1 | k2)) continue;
+                const cx x[4] = {a[i], a[i | k1], a[i | k2], a[i | k1 | k2]};
+                if (g.kind == F_DAMP1) {
+                    a[i] = x[0] + g.f[0] * x[3];
+                    a[i | k1] = g.f[1] * x[1];
+                    a[i | k2] = g.f[1] * x[2];
+                    a[i | k1 | k2] = g.f[2] * x[3];
+                } else {
+                    a[i] = g.f[0] * x[0] + g.f[1] * x[3];
+                    a[i | k1] = g.f[2] * x[1] + g.f[3] * x[2];
+                    a[i | k2] = g.f[2] * x[2] + g.f[3] * x[1];
+                    a[i | k1 | k2] = g.f[0] * x[3] + g.f[1] * x[0];
+                }
+            }
+            break;
+        }
         case F_DEPOL2: {
             // every amplitude scales; the 4 of a group with ket = bra on both
             // qubits then share a multiple of their sum
@@ -320,7 +339,8 @@ static GOp randomGate(Rng& r, int n, bool dens, int hot) {
             break;
         }
         default: {
-            g.kind = r.below(2) ? F_DEPOL1 : F_DEPH1;
+            const int channel = r.below(4);
+            g.kind = channel == 0 ? F_DEPOL1 : channel == 1 ? F_DEPH1 : channel == 2 ? F_DAMP1 : F_PAULIS1;
             const int q = r.below(n / 2);
             g.t1 = q;
             g.t2 = q + n / 2;
@@ -328,6 +348,12 @@ static GOp randomGate(Rng& r, int n, bool dens, int hot) {
             g.f[0] = g.kind == F_DEPOL1 ? 1 - 2 * p / 3 : 1 - 2 * p;
             g.f[1] = 2 * p / 3;
             g.f[2] = 1 - 4 * p / 3;
+            g.f[3] = p / 3;
+            if (g.kind == F_DAMP1) {
+                g.f[0] = p;
+                g.f[1] = std::sqrt(1 - p);
+                g.f[2] = 1 - p;
+            }
             break;
         }
     }

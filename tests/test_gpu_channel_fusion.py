@@ -114,3 +114,31 @@ def test_channels_in_mfma_blocks(api, min_gates):
         api.gpu().qa_setFusionBlocks(0)
         api.set_fusion(bool(before[0]), *before[1:])
     assert rel(got, want) <= 8 * 2.0 ** -24 * len(c.ops)
+
+
+@pytest.mark.parametrize("kind", ["DAMP", "PAULIS"])
+def test_channels_keep_infinite_amplitudes(api, kind):
+    """One infinite amplitude: a channel in a pass touches what its own kernel
+    touches, where a matrix would make NaN of the whole group."""
+    print(f"[gpu] infinite amplitudes under {kind}", flush=True)
+    before = api.get_fusion()
+    n = 5
+    rho = qc.random_state(n, 91, True)
+    rho[0b00111_10110] = np.inf
+    c = qc.Circuit(n, True, [], ("given",), "infinite")
+    for q in (1, 0, 1, 3, 1):
+        c.ops.append((kind, q, *([0.2] if kind == "DAMP" else [0.1, 0.2, 0.05])))
+    got = []
+    try:
+        for enabled in (False, True):
+            api.set_fusion(enabled, 8, 3, 512)
+            q = api.createDensityQureg(n)
+            api.set_amps(q, rho)
+            q, _ = qc.run(c, q)
+            got.append(api.get_amps(q))
+            api.destroyQureg(q)
+    finally:
+        api.set_fusion(bool(before[0]), *before[1:])
+    assert np.count_nonzero(np.isnan(got[0].real)) == 0
+    assert np.allclose(got[1].real, got[0].real, rtol=1e-13, atol=1e-15)
+    assert np.array_equal(np.isfinite(got[1]), np.isfinite(got[0]))
