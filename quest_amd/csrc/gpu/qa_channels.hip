@@ -282,24 +282,16 @@ int qa_densmatr_twoQubitDephasing(void* amps, int prec, int N, int q1, int q2, d
     QA_ARG_CHECK(q1 >= 0 && q1 < N && q2 >= 0 && q2 < N && q1 != q2, "%s: bad qubits", __func__);
     uint64_t num = 1ull << (2 * N);
     double term = -4 * prob / 3;  // util_getTwoQubitDephasingTerm
-    if (!fuse::exactMode() && 1 + term >= 0 && fuse::enabledFor(amps, prec, 2 * N)) {
-        // f = 1 + term where either qubit's ket and bra differ: the product of
-        // sqrt(f) for each of qubit 1's, qubit 2's and their joint parity,
-        // two of which are odd in each of those cases.  Queued so, the channel
-        // is diagonal, needs no qubit in the tile, and merges with the gates
-        // around it (a pass of its own costs 0.27 ms at 13 qubits)
-        const uint64_t a = (1ull << q1) | (1ull << (q1 + N)), b = (1ull << q2) | (1ull << (q2 + N));
-        for (uint64_t m : {a, b, a | b}) {
-            fuse::GOp op;
-            op.kind = fuse::F_PARITY;
-            op.m1 = m;
-            op.f[0] = 1;
-            op.f[2] = std::sqrt(1 + term);
-            bool accepted = false;
-            const int rc = fuse::enqueue(amps, prec, 2 * N, op, accepted);
-            if (rc != QA_OK) return rc;
-        }
-        return QA_OK;
+    if (!fuse::exactMode()) {
+        // as one diagonal op the channel needs no qubit in the tile (a pass of
+        // its own costs 0.27 ms at 13 qubits), and it multiplies each
+        // amplitude once, by the factor of the kernel below
+        fuse::GOp op;
+        op.kind = fuse::F_DEPH2;
+        op.m1 = (1ull << q1) | (1ull << (q1 + N));
+        op.m2 = (1ull << q2) | (1ull << (q2 + N));
+        op.f[0] = prec == QA_FP64 ? 1 + term : (double)(1.0f + (float)term);
+        QA_TRY_FUSE(amps, prec, 2 * N, op);
     }
     QA_FLUSH_ALL();
     QA_DISPATCH(prec, (k_dephase2<T><<<gridFor(num), BLOCK, 0, stream()>>>((T*)amps, num, q1, q1 + N, q2,

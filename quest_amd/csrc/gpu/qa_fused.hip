@@ -207,6 +207,11 @@ TOp toTile(const GOp& g, const Layout& L) {
     } else if (g.kind == F_PAULI) {
         t.b[4] = jm2;
         t.b[5] = gm2;
+    } else if (g.kind == F_DEPH2) {
+        t.b[4] = jm1;
+        t.b[5] = gm1;
+        t.b[6] = jm2;
+        t.b[7] = gm2;
     }
     // DENSE2: matrix elements 4..15 (the first 4 are in b)
     if (g.kind == F_DENSE2) std::memcpy(t.fx, g.f + 8, 24 * sizeof(double));
@@ -722,7 +727,7 @@ uint64_t supportMask(const GOp& g) {
         case F_DENSE1V: m |= g.m1; break;
         case F_DIAG1: m |= 1ull << g.t1; break;
         case F_PARITY: m |= g.m1; break;
-        case F_PAULI: m |= g.m1 | g.m2; break;
+        case F_PAULI: case F_DEPH2: m |= g.m1 | g.m2; break;
         default: break;
     }
     return m;
@@ -841,6 +846,12 @@ bool applySmall(const GOp& g, const int* q, int nq, std::complex<double>* v) {
             const uint32_t k1 = 1u << bitOf(g.t1), k2 = 1u << bitOf(g.t2);
             for (int j = 0; j < D; j++)
                 if (((j & k1) != 0) != ((j & k2) != 0)) v[j] *= g.f[0];
+            break;
+        }
+        case F_DEPH2: {
+            const uint32_t a = loc(g.m1), b = loc(g.m2);
+            for (int j = 0; j < D; j++)
+                if ((__builtin_popcount(j & a) | __builtin_popcount(j & b)) & 1) v[j] *= g.f[0];
             break;
         }
         case F_DAMP1: case F_PAULIS1: {
@@ -1289,6 +1300,7 @@ double opFlops(const GOp& g, int n) {
         case F_PAULI: perAmp = 14; break;    // multiply + multiply-add per amplitude
         case F_DEPOL1: perAmp = 4; break;    // 16 per 4 amplitudes
         case F_DEPH1: perAmp = 1; break;     // 4 per 4 amplitudes
+        case F_DEPH2: perAmp = 1.5; break;   // 2 on 3 of 4 amplitudes
         case F_DAMP1: perAmp = 2.5; break;   // 10 per 4 amplitudes
         case F_PAULIS1: perAmp = 6; break;   // a multiply and a multiply-add each
         case F_DEPOL2: perAmp = 3; break;    // one multiply each, 4 of 16 also share a sum

@@ -18,6 +18,7 @@ struct GOp {
     double f[32] = {0};              // matrix / factors (re, im interleaved); DENSE1V: one 2x2
                                      // matrix per value w of the (at most 2) variant qubits, at
                                      // f[8w], bit b of w = the b-th lowest variant qubit
+    // DEPH2: f[0] where the index has an odd number of the bits of m1, or of m2
     // DEPOL2: targs = the two ket qubits, then their bra qubits
     // DENSEN: targets (matrix index bit b <-> targs[b]), and the row-major
     // 2^n x 2^n matrix {re, im} in device memory staged by stageMatrix

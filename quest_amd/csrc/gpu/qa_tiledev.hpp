@@ -62,6 +62,8 @@ static_assert(sizeof(TOpHead) == 64, "op header is one 64-byte scalar load");
 //     parity mask (PARITY) or the maskYZ bits (PAULI) outside the
 //     registers, b[5] = its non-local part
 //   DEPOL1: b[0..2] = c1, c2, c3;  DEPH1: b[0] = factor
+//   DEPH2: b[0] = factor, rm1, b[4], b[5] the masks of one qubit's ket and bra
+//     as for a PARITY, rm2, b[6], b[7] the other's
 //   DAMP1: b[0..2] = prob, c1, c2;  PAULIS1: b[0..3] = fAA, fBB, fAB, fBA
 //   DEPOL2: b[0..2] = c1 - c2, c2, 1 + c3; rb1 = the register bit that is the
 //     other half (bra or ket) of register bit 0's qubit
@@ -496,6 +498,21 @@ __device__ __forceinline__ void regDeph1(ct<T>* r, const double* f) {
     }
 }
 
+// two-qubit dephasing: f where either qubit's ket and bra differ; parA and
+// parB are the qubits' parities over the bits outside the registers
+template <typename T>
+__device__ __forceinline__ void regDeph2(ct<T>* r, const OpRegs& o, uint32_t jb, uint64_t base) {
+    const T f = (T)o.f[0];
+    const uint64_t jmB = (uint64_t)__double_as_longlong(o.f[6]), gmB = (uint64_t)__double_as_longlong(o.f[7]);
+    const int parA = parity64((jb & o.jm) ^ (base & o.gm)), parB = parity64((jb & jmB) ^ (base & gmB));
+#pragma unroll
+    for (int v = 0; v < RA; v++) {
+        const bool differ = ((__popc((uint32_t)v & o.h.rm1) & 1) ^ parA) | ((__popc((uint32_t)v & o.h.rm2) & 1) ^ parB);
+        const T x = differ ? f : (T)1;
+        r[v] = ct<T>{r[v].re * x, r[v].im * x};
+    }
+}
+
 template <typename T, int B1, int B2>
 __device__ __forceinline__ void regDamp1(ct<T>* r, const double* f) {
     const T prob = (T)f[0], c1 = (T)f[1], c2 = (T)f[2];
@@ -864,6 +881,9 @@ __device__ __forceinline__ void applyOp(ct<T>* r, const TOp* __restrict__ op, co
                 switch (h.rb1 * RB + h.rb2) { QA_CHAN_CASES(regDeph1) }
             }
             break;
+        case F_DEPH2:
+            if constexpr (!SV) regDeph2<T>(r, o, jb, base);
+            break;
         case F_DAMP1:
             if constexpr (!SV) {
                 switch (h.rb1 * RB + h.rb2) { QA_CHAN_CASES(regDamp1) }
@@ -948,6 +968,8 @@ __device__ __forceinline__ void applyFixed(ct<T>* r, const TOp* __restrict__ op,
         regDepol1<T, RB1, RB2>(r, f);
     } else if constexpr (KIND == F_DEPH1) {
         regDeph1<T, RB1, RB2>(r, f);
+    } else if constexpr (KIND == F_DEPH2) {
+        regDeph2<T>(r, o, jb, base);
     } else if constexpr (KIND == F_DAMP1) {
         regDamp1<T, RB1, RB2>(r, f);
     } else if constexpr (KIND == F_PAULIS1) {

@@ -148,6 +148,10 @@ static void apply(const GOp& g, std::vector<cx>& a) {
                 if (((i & k1) != 0) != ((i & k2) != 0)) a[i] *= g.f[0];
             break;
         }
+        case F_DEPH2:
+            for (uint64_t i = 0; i < N; i++)
+                if (parity(i & g.m1) || parity(i & g.m2)) a[i] *= g.f[0];
+            break;
         case F_DAMP1: case F_PAULIS1: {
             const uint64_t k1 = 1ull << g.t1, k2 = 1ull << g.t2;
             for (uint64_t i = 0; i < N; i++) {
@@ -255,6 +259,15 @@ static GOp randomGate(Rng& r, int n, bool dens, int hot) {
         do g.targs[1] = r.below(n / 2); while (g.targs[1] == g.targs[0]);
         g.targs[2] = g.targs[0] + n / 2;
         g.targs[3] = g.targs[1] + n / 2;
+        if (r.below(3) == 0) {
+            // or two-qubit dephasing
+            g.kind = F_DEPH2;
+            g.m1 = (1ull << g.targs[0]) | (1ull << g.targs[2]);
+            g.m2 = (1ull << g.targs[1]) | (1ull << g.targs[3]);
+            g.numTargs = 0;
+            g.f[0] = 0.5 * (r.unit() + 1);
+            return g;
+        }
         const double p = r.below(2) ? 15.0 / 16 : 0.05 * (r.unit() + 1);
         g.f[0] = 1 - 16 * p / 15;
         g.f[1] = 4 * p / 15;

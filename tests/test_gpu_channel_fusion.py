@@ -116,7 +116,34 @@ def test_channels_in_mfma_blocks(api, min_gates):
     assert rel(got, want) <= 8 * 2.0 ** -24 * len(c.ops)
 
 
-@pytest.mark.parametrize("kind", ["DAMP", "PAULIS"])
+@pytest.mark.parametrize("prec", [2, 1])
+@pytest.mark.parametrize("jit", [0, 2])
+def test_two_qubit_dephasing_rounds_once(api, prec, jit):
+    """In a pass, on qubits in and outside the registers and the tile, the
+    channel multiplies each amplitude once and by the factor of its own kernel:
+    the results are equal, bit for bit."""
+    print(f"[gpu] two-qubit dephasing in passes prec={prec} jit={jit}", flush=True)
+    before = api.get_fusion()
+    n = 7
+    c = qc.Circuit(n, True, [], ("random", 93), "dephasing")
+    for a, b, p in [(0, 1, 0.3), (0, 6, 0.11), (5, 6, 0.75), (2, 4, 0.05), (3, 6, 0.4), (1, 5, 0.2)]:
+        c.ops.append(("DEPH2", a, b, p))
+    got = []
+    try:
+        for enabled in (False, True):
+            api.set_fusion(enabled, 8, 3, 512)
+            api.set_fusion_jit(jit, 1)
+            q = api.createCustomPrecisionQureg(n, 1, prec)
+            q, _ = qc.run(c, q)
+            got.append(api.get_amps(q))
+            api.destroyQureg(q)
+    finally:
+        api.set_fusion_jit(1, 2)
+        api.set_fusion(bool(before[0]), *before[1:])
+    assert np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("kind", ["DAMP", "PAULIS", "DEPH2"])
 def test_channels_keep_infinite_amplitudes(api, kind):
     """One infinite amplitude: a channel in a pass touches what its own kernel
     touches, where a matrix would make NaN of the whole group."""
@@ -127,7 +154,7 @@ def test_channels_keep_infinite_amplitudes(api, kind):
     rho[0b00111_10110] = np.inf
     c = qc.Circuit(n, True, [], ("given",), "infinite")
     for q in (1, 0, 1, 3, 1):
-        c.ops.append((kind, q, *([0.2] if kind == "DAMP" else [0.1, 0.2, 0.05])))
+        c.ops.append((kind, q, *{"DAMP": [0.2], "PAULIS": [0.1, 0.2, 0.05], "DEPH2": [4, 0.2]}[kind]))
     got = []
     try:
         for enabled in (False, True):
