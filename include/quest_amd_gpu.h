@@ -380,9 +380,8 @@ int qa_densmatr_calcExpecPauliStr(const void* amps, int prec, int numQubitsN,
    bit masks, coeffs complex (re, im interleaved).  Strings that share their
    X/Y mask mix the same amplitude pairs; up to 8 of them are reduced in one
    read of the state, each term's value bitwise equal to
-   qa_statevec_calcExpecPauliStr's.  From 22 qubits up to 4 such groups share
-   one read, and a term's value equals the single string's up to the rounding
-   of FP64 sums.  The weighted sum is taken in term order.  termValues (2 doubles per term, may be NULL) receives every <P_t>. */
+   qa_statevec_calcExpecPauliStr's.  The weighted sum is taken in term
+   order.  termValues (2 doubles per term, may be NULL) receives every <P_t>. */
 int qa_statevec_calcExpecPauliStrSum(const void* amps, int prec, int numQubits, int64_t numTerms,
                                      const uint64_t* maskX, const uint64_t* maskY, const uint64_t* maskZ,
                                      const double* coeffs, double* termValues, double* out);

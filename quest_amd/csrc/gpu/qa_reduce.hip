@@ -36,11 +36,11 @@ constexpr int RED_BLOCKS = 1024;
 // slot's values, then its ticket.  A slot comes round again after LAND_SLOTS
 // reductions, each of which its caller has waited for.
 constexpr int LAND_SLOTS = 256;
-constexpr int LAND_VALUES = 16;
+constexpr int LAND_VALUES = 20;
 struct LandSlot {
     double v[LAND_VALUES];
     uint64_t ticket;
-    uint64_t pad[7];
+    uint64_t pad[11];
 };
 LandSlot* g_land = nullptr;
 std::atomic<uint64_t> g_ticket{0};
@@ -138,9 +138,9 @@ __global__ void __launch_bounds__(BLOCK) k_reduce(F f, uint64_t numWork, double*
 }
 
 // merges numParts partials of nv <= LAND_VALUES values (a wave per value, in
-// a fixed order) and lands them
+// a fixed order) and lands them; pairs: a value as (s, c), all s first
 __device__ __forceinline__ void mergePartials(const double* __restrict__ partials, int numParts, int nv,
-                                              const Ticket& ticket) {
+                                              const Ticket& ticket, bool pairs = false) {
     __shared__ double out[LAND_VALUES];
     const int lane = threadIdx.x & 63;
     for (int v = threadIdx.x >> 6; v < nv; v += BLOCK / 64) {
@@ -148,10 +148,13 @@ __device__ __forceinline__ void mergePartials(const double* __restrict__ partial
         for (int p = lane; p < numParts; p += 64)
             kmerge(acc, KB{partials[(p * nv + v) * 2], partials[(p * nv + v) * 2 + 1]});
         waveMerge(acc);
-        if (lane == 0) out[v] = acc.s + acc.c;
+        if (lane == 0) {
+            out[v] = pairs ? acc.s : acc.s + acc.c;
+            if (pairs) out[nv + v] = acc.c;
+        }
     }
     __syncthreads();
-    if (threadIdx.x == 0) landValues(ticket, out, nv);
+    if (threadIdx.x == 0) landValues(ticket, out, pairs ? 2 * nv : nv);
 }
 
 __global__ void __launch_bounds__(BLOCK) k_finalize(const double* __restrict__ partials, int numParts, int nv,
@@ -384,13 +387,15 @@ struct FDensExpecZ {
 // Without X or Y a term is sign |a_n|^2.  A string's sum is bitwise the same
 // alone or in a group read by itself.
 constexpr int GROUP_STRINGS = 8;
+constexpr int GROUP_VALUES = GROUP_STRINGS + 2;  // of one partial, at most
 struct PauliGroup {
     uint64_t maskXY, topLow;  // topLow: the bits below the top X/Y bit
     uint64_t maskYZ[GROUP_STRINGS];
     uint64_t odd;             // bit t: string t has an odd number of Y
     uint64_t numWork;
     int blocks, numStrings;
-    int nv, pad;              // values of one partial: numStrings, or more
+    int nv;                   // values of one partial: numStrings, or more
+    int pairs;                // a shared read: values land as (s, c), all s first
     Ticket ticket;
 };
 template <typename T, int NT>
@@ -432,12 +437,12 @@ __global__ void __launch_bounds__(BLOCK) k_pauliGroups(const T* __restrict__ a, 
     f.a = a;
     f.g = g;
     reduceTerms<NT>(f, g.numWork, blockIdx.x, (unsigned)g.blocks,
-                    partials + (size_t)blockIdx.y * RED_BLOCKS * GROUP_STRINGS * 2, g.blocks == 1, g.ticket);
+                    partials + (size_t)blockIdx.y * RED_BLOCKS * GROUP_VALUES * 2, g.blocks == 1, g.ticket);
 }
 __global__ void __launch_bounds__(BLOCK) k_finalizeGroups(PauliGroups gs, const double* __restrict__ partials) {
     const PauliGroup& g = gs.g[blockIdx.x];
     if (g.blocks == 1) return;
-    mergePartials(partials + (size_t)blockIdx.x * RED_BLOCKS * GROUP_STRINGS * 2, g.blocks, g.nv, g.ticket);
+    mergePartials(partials + (size_t)blockIdx.x * RED_BLOCKS * GROUP_VALUES * 2, g.blocks, g.nv, g.ticket, g.pairs);
 }
 
 // G = 2..4 groups with linearly independent X/Y masks in one read of the
@@ -445,25 +450,40 @@ __global__ void __launch_bounds__(BLOCK) k_finalizeGroups(PauliGroups gs, const 
 // the masks' pivot bits clear, and finds every group's pairs among them, v and
 // v with bit g flipped.  Group after group the state would be read G times,
 // which is all that such a sum costs on a state larger than the caches.  The
-// signs over v are uniform, so a string adds its 2^(G-1) pairs with one
-// multiply-add by +-1 each before the compensated sum.  25 qubits complex128,
-// four groups of 5 strings: 128 us, 4.2 TB/s (92 us for each group alone); with
-// 8 strings the arithmetic is the bound.
+// terms are those of FPauliGroup, bit for bit (the first of a pair is the one
+// with the mask's top bit, a pivot, clear), and each is added compensated.
+// A string's sum (s, c) goes to the host as it is, with the sum of its terms'
+// magnitudes: see settled().  Bound by arithmetic where groups have several
+// strings, 9 FP64 operations a pair and string: 25 qubits complex128, four
+// groups of 5 strings 193 us, of one 119 us (a read for each group: 4 x 92).
+__device__ __forceinline__ double flipIf(double x, uint32_t signBit) {
+    return __longlong_as_double(__double_as_longlong(x) ^ (long long)((uint64_t)signBit << 32));
+}
+// kadd of sign * v, sign being 1 or -1
+__device__ __forceinline__ void kaddSigned(KB& a, double v, double sign) {
+    const double t = fmaT(v, sign, a.s), bb = t - a.s;
+    a.c += (a.s - (t - bb)) + fmaT(v, sign, -bb);
+    a.s = t;
+}
 struct PauliSpan {
     PauliGroup g[4];
     uint64_t signs[4];  // byte t: bit p the sign of string t's pair p against the thread's own
+    uint32_t swapped[4];  // bit p: the second of pair p has the top bit clear
     InsertSpec pivots;
     uint64_t numWork;
 };
 template <typename T, int G, int NT>
-__global__ void __launch_bounds__(BLOCK) k_pauliSpan(const T* __restrict__ a, PauliSpan s,
+__global__ void __launch_bounds__(BLOCK, 2) k_pauliSpan(const T* __restrict__ a, PauliSpan s,
                                                     double* __restrict__ partials) {
     constexpr int V = 1 << G;
     KB acc[G][NT];
+    double magnitude[G][2];  // of the even and the odd strings' terms
 #pragma unroll
-    for (int g = 0; g < G; g++)
+    for (int g = 0; g < G; g++) {
+        magnitude[g][0] = magnitude[g][1] = 0;
 #pragma unroll
         for (int t = 0; t < NT; t++) acc[g][t] = KB{0, 0};
+    }
     uint64_t at[V];
 #pragma unroll
     for (int v = 0; v < V; v++) {
@@ -485,44 +505,63 @@ __global__ void __launch_bounds__(BLOCK) k_pauliSpan(const T* __restrict__ a, Pa
                 const int v = ((p >> g) << (g + 1)) | (p & ((1 << g) - 1));
                 const cd y = x[v], z = x[v | (1 << g)];
                 re[p] = fmaT(y.re, z.re, y.im * z.im);
-                im[p] = fmaT(y.re, z.im, -(y.im * z.re));
+                const double yz = fmaT(y.re, z.im, -(y.im * z.re)), zy = fmaT(z.re, y.im, -(z.im * y.re));
+                im[p] = (s.swapped[g] >> p) & 1u ? zy : yz;
+                magnitude[g][0] += fabs(re[p]);
+                magnitude[g][1] += fabs(im[p]);
             }
 #pragma unroll
             for (int t = 0; t < NT; t++) {
+                // the thread's own sign is taken by the accumulator, which
+                // leaves the pairs' signs uniform: operands of the additions
                 const uint32_t signs = (uint32_t)(s.signs[g] >> (8 * t));
-                double sum = 0;
-                if ((s.g[g].odd >> t) & 1ull) {
+                const uint32_t own = parity64(n & s.g[g].maskYZ[t]) ? 0x80000000u : 0u;
+                KB sum = {flipIf(acc[g][t].s, own), flipIf(acc[g][t].c, own)};
+                const bool odd = (s.g[g].odd >> t) & 1ull;
 #pragma unroll
-                    for (int p = 0; p < V / 2; p++) sum = fmaT(im[p], (signs >> p) & 1u ? -1.0 : 1.0, sum);
-                } else {
-#pragma unroll
-                    for (int p = 0; p < V / 2; p++) sum = fmaT(re[p], (signs >> p) & 1u ? -1.0 : 1.0, sum);
-                }
-                const uint64_t yz = s.g[g].maskYZ[t];
-                kadd(acc[g][t], parity64(n & yz) ? -sum : sum);
+                for (int p = 0; p < V / 2; p++)
+                    kaddSigned(sum, odd ? im[p] : re[p], (signs >> p) & 1u ? -1.0 : 1.0);
+                acc[g][t] = KB{flipIf(sum.s, own), flipIf(sum.c, own)};
             }
         }
     }
 #pragma unroll
     for (int g = 0; g < G; g++) {
-        blockMerge<NT>(acc[g]);
+        KB sums[NT + 2];
+#pragma unroll
+        for (int t = 0; t < NT; t++) sums[t] = acc[g][t];
+        sums[NT] = KB{magnitude[g][0], 0};
+        sums[NT + 1] = KB{magnitude[g][1], 0};
+        blockMerge<NT + 2>(sums);
         if (threadIdx.x == 0) {
-            if (gridDim.x == 1) {
-                double out[NT];
+            double* dst =
+                partials + (size_t)g * RED_BLOCKS * GROUP_VALUES * 2 + (size_t)blockIdx.x * (NT + 2) * 2;
 #pragma unroll
-                for (int t = 0; t < NT; t++) out[t] = acc[g][t].s + acc[g][t].c;
-                landValues(s.g[g].ticket, out, NT);
-            } else {
-                double* dst = partials + (size_t)g * RED_BLOCKS * GROUP_STRINGS * 2 + (size_t)blockIdx.x * NT * 2;
-#pragma unroll
-                for (int t = 0; t < NT; t++) {
-                    dst[2 * t] = acc[g][t].s;
-                    dst[2 * t + 1] = acc[g][t].c;
-                }
+            for (int t = 0; t < NT + 2; t++) {
+                dst[2 * t] = sums[t].s;
+                dst[2 * t + 1] = sums[t].c;
             }
         }
         __syncthreads();  // the next group's merge reuses the workgroup's LDS
     }
+}
+
+// The value of a sum that a shared read left as (s, c), if it is certain that
+// the string's own read gives the same double.
+// Both add the same terms, exactly but for the rounding of the compensations:
+// an accumulator of k terms holds a compensation of at most k u A (u = 2^-53, A
+// the sum of its terms' magnitudes), rounded k times, and D merges round the
+// sums of compensations twice each, so that s + c is within 2 (k + D)^2 u^2 A
+// of the exact sum of the terms.  The two are then apart by at most delta =
+// 4 (k + D)^2 u^2 A, k being the longer chain's, here taken twice, and round to
+// the same double when the interval around s + c does.  A sum that is zero but
+// for rounding is not settled, nor is one with infinities or NaN.
+bool settled(double s, double c, double magnitude, uint64_t chain, double& value) {
+    constexpr double MERGES = 48;  // 6 over a wave, 3 waves, 16 partials a lane, 6 more, and some
+    const double k = (double)chain + MERGES, delta = 8 * k * k * 0x1p-106 * magnitude;
+    const double lo = s + (c - delta), hi = s + (c + delta);
+    value = hi;
+    return lo == hi;
 }
 
 template <typename T>
@@ -1074,10 +1113,11 @@ int launchGroups(const T* a, PauliGroups& gs, int from, int to, double* scratch)
     for (int i = from; i < to; i++) most = std::max(most, gs.g[i].numStrings);
     for (int i = from; i < to; i++) {
         gs.g[i].nv = most;
+        gs.g[i].pairs = 0;
         sub.g[i - from] = gs.g[i];
         maxBlocks = std::max(maxBlocks, gs.g[i].blocks);
     }
-    double* dst = scratch + (size_t)from * RED_BLOCKS * GROUP_STRINGS * 2;
+    double* dst = scratch + (size_t)from * RED_BLOCKS * GROUP_VALUES * 2;
     const dim3 grid((unsigned)maxBlocks, (unsigned)(to - from), 1);
     switch (most) {
 #define QA_NV(NV) \
@@ -1090,13 +1130,21 @@ int launchGroups(const T* a, PauliGroups& gs, int from, int to, double* scratch)
 }
 
 // one launch of groups gs.g[from, from + num), num = 2..4 with independent
-// masks, in one read
+// masks, in one read; chain: the most terms that one accumulator adds
 template <typename T>
-int launchSpanGroups(const T* a, int nq, PauliGroups& gs, int from, int num, double* scratch) {
+int launchSpanGroups(const T* a, int nq, PauliGroups& gs, int from, int num, double* scratch, uint64_t& chain) {
     PauliSpan s;
+    // the first amplitude of pair p of group g, against the thread's own: the
+    // masks selected by p with a zero inserted at bit g
+    auto firstOf = [&](int g, int p) {
+        const int v = ((p >> g) << (g + 1)) | (p & ((1 << g) - 1));
+        uint64_t at = 0;
+        for (int b = 0; b < num; b++)
+            if ((v >> b) & 1) at ^= s.g[b].maskXY;
+        return at;
+    };
     int most = 1;
     for (int i = 0; i < num; i++) most = std::max(most, gs.g[from + i].numStrings);
-    if (most > 2 && most % 2) most++;  // kernels for 1, 2, 4, 6 and 8 strings a group
     // each mask less the pivots (highest bits) of those before it
     uint64_t lead[4], pivots = 0;
     for (int i = 0; i < num; i++) {
@@ -1111,35 +1159,39 @@ int launchSpanGroups(const T* a, int nq, PauliGroups& gs, int from, int num, dou
     for (int q = 0; q < nq; q++)
         if ((pivots >> q) & 1ull) s.pivots.pos[s.pivots.num++] = q;
     s.numWork = 1ull << (nq - num);
-    // no more workgroups than are resident (16 accumulators and more: 2 waves per SIMD)
-    const int resident = num * most >= 16 ? RED_BLOCKS / 2 : RED_BLOCKS;
-    const int blocks = (int)std::min<uint64_t>((uint64_t)resident, (s.numWork + BLOCK - 1) / BLOCK);
+    // as many workgroups as are resident (2 waves per SIMD)
+    const int blocks = (int)std::min<uint64_t>(RED_BLOCKS / 2, (s.numWork + BLOCK - 1) / BLOCK);
     for (int i = 0; i < num; i++) {
-        gs.g[from + i].nv = most;
+        gs.g[from + i].nv = most + 2;
+        gs.g[from + i].pairs = 1;
         gs.g[from + i].blocks = blocks;
         s.g[i] = gs.g[from + i];
     }
+    chain = (s.numWork / ((uint64_t)blocks * BLOCK) + 1) << (num - 1);
     for (int g = 0; g < num; g++) {
         s.signs[g] = 0;
+        s.swapped[g] = 0;
+        const uint64_t top = s.g[g].topLow + 1;
+        for (int p = 0; p < (1 << num) / 2; p++)
+            s.swapped[g] |= (firstOf(g, p) & top) ? 1u << p : 0u;
         for (int t = 0; t < s.g[g].numStrings; t++) {
             const uint64_t odd = (s.g[g].odd >> t) & 1ull;
             for (int p = 0; p < (1 << num) / 2; p++) {
-                // the pair's first amplitude: p with a zero inserted at bit g
-                const int v = ((p >> g) << (g + 1)) | (p & ((1 << g) - 1));
-                uint64_t at = 0;
-                for (int b = 0; b < num; b++)
-                    if ((v >> b) & 1) at ^= s.g[b].maskXY;
-                // an even string's sign is the first amplitude's, an odd one's the second's
-                const uint64_t par = (uint64_t)(__builtin_popcountll(at & s.g[g].maskYZ[t]) & 1);
-                s.signs[g] |= (par ^ odd) << (8 * t + p);
+                // an even string's sign is that of either amplitude, an odd one's
+                // that of the amplitude with the top bit set
+                const uint64_t par = (uint64_t)(__builtin_popcountll(firstOf(g, p) & s.g[g].maskYZ[t]) & 1);
+                const uint64_t swapped = (s.swapped[g] >> p) & 1u;
+                s.signs[g] |= (par ^ (odd & ~swapped)) << (8 * t + p);
             }
         }
     }
-    double* dst = scratch + (size_t)from * RED_BLOCKS * GROUP_STRINGS * 2;
+    double* dst = scratch + (size_t)from * RED_BLOCKS * GROUP_VALUES * 2;
     switch (num * 16 + most) {
 #define QA_SPAN(G, NT) \
     case G * 16 + NT: k_pauliSpan<T, G, NT><<<blocks, BLOCK, 0, stream()>>>(a, s, dst); break
-#define QA_SPANS(G) QA_SPAN(G, 1); QA_SPAN(G, 2); QA_SPAN(G, 4); QA_SPAN(G, 6); QA_SPAN(G, 8)
+#define QA_SPANS(G)                                             \
+    QA_SPAN(G, 1); QA_SPAN(G, 2); QA_SPAN(G, 3); QA_SPAN(G, 4); \
+    QA_SPAN(G, 5); QA_SPAN(G, 6); QA_SPAN(G, 7); QA_SPAN(G, 8)
         QA_SPANS(2); QA_SPANS(3); QA_SPANS(4);
 #undef QA_SPANS
 #undef QA_SPAN
@@ -1161,18 +1213,29 @@ bool independent(const uint64_t* masks, int num, uint64_t mask) {
 
 // Sums over states of at least this many qubits read the state once for up to
 // 4 groups (k_pauliSpan).  One call, a read per four groups against a read per
-// group (us, complex128; groups x strings):
-//   qubits   2x1        4x1        4x4        4x8        8x4
-//   20       19 / 18    18 / 23    24 / 27    35 / 32    38 / 33
-//   22       27 / 31    30 / 49    36 / 62    71 / 72    58 / 89
-//   24       57 / 90    56 / 168   64 / 182   139 / 195  128 / 327
-// (complex64 at 22: 28 / 33 for 4x1, 53 / 68 for 8x4)
+// group (us, random states; groups x strings):
+//   complex128   2x1        4x1        4x4        4x5        4x8        8x4
+//   20 qubits    18 / 16    19 / 20    28 / 26    31 / 29    43 / 33    44 / 32
+//   21           18 / 25    22 / 34    35 / 36    39 / 45    58 / 50    60 / 53
+//   22           26 / 35    29 / 47    46 / 52    50 / 61    73 / 69    77 / 90
+//   23           35 / 48    41 / 84    62 / 90    69 / 98    104 / 115  107 / 168
+//   24           52 / 88    58 / 164   92 / 187   106 / 185  168 / 197  177 / 332
+//   complex64
+//   21           18 / 20    22 / 26    35 / 32    38 / 40    54 / 48    56 / 46
+//   22           22 / 25    26 / 31    43 / 43    48 / 53    70 / 67    72 / 68
+//   23           29 / 33    35 / 47    60 / 65    67 / 78    99 / 104   104 / 115
+//   24           41 / 51    48 / 79    90 / 107   106 / 131  161 / 182  172 / 193
+// A group with a sum that is not settled (zero but for rounding, which
+// symmetries of a state bring about) is read once more: at worst the two
+// add up, 26 qubits complex128 4x5 strings of zero sum 1057 us, alone 715.
 constexpr int SPAN_MIN_QUBITS = 22;
 
 // The values of numTerms Pauli strings, (re, im) each, in vals: strings are
 // grouped by X/Y mask (of at most GROUP_STRINGS, in ascending mask order, each
 // in term order), and each group is one read of the state or shares one with
-// up to three others.  Up to MAX_GROUPS groups are launched together and then
+// up to three others; where a shared read leaves a last bit open, the group is
+// read by itself too, so that a string's value is that of its own read
+// whatever it is summed with.  Up to MAX_GROUPS groups are launched together and then
 // waited for.
 template <typename T>
 int expecStrings(const T* a, int nq, int64_t numTerms, const uint64_t* maskX, const uint64_t* maskY,
@@ -1200,6 +1263,7 @@ int expecStrings(const T* a, int nq, int64_t numTerms, const uint64_t* maskX, co
     while (!alone.empty() || !rest.empty()) {
         PauliGroups gs;
         int64_t first[MAX_GROUPS];
+        uint64_t chains[MAX_GROUPS];
         int num = 0, rc = QA_OK;
         auto take = [&](const Group& x) {
             PauliGroup& g = gs.g[num];
@@ -1220,7 +1284,7 @@ int expecStrings(const T* a, int nq, int64_t numTerms, const uint64_t* maskX, co
         };
         if (!scratch) {
             const size_t groups = std::min<size_t>(MAX_GROUPS, alone.size() + rest.size());
-            scratch = devScratch(groups * RED_BLOCKS * GROUP_STRINGS * 2);
+            scratch = devScratch(groups * RED_BLOCKS * GROUP_VALUES * 2);
             if (!scratch || !g_land) {
                 setError("reduction scratch unavailable");
                 return QA_ERR_OOM;
@@ -1240,8 +1304,10 @@ int expecStrings(const T* a, int nq, int64_t numTerms, const uint64_t* maskX, co
                 }
             }
             rest.swap(later);
-            rc = n > 1 ? launchSpanGroups(a, nq, gs, from, n, scratch) : launchGroups(a, gs, from, num, scratch);
+            uint64_t chain = 0;
+            rc = n > 1 ? launchSpanGroups(a, nq, gs, from, n, scratch, chain) : launchGroups(a, gs, from, num, scratch);
             if (rc != QA_OK) return rc;
+            for (int i = from; i < num; i++) chains[i] = chain;
         }
         const int from = num;
         while (!alone.empty() && num < MAX_GROUPS) {
@@ -1258,9 +1324,22 @@ int expecStrings(const T* a, int nq, int64_t numTerms, const uint64_t* maskX, co
         }
         for (int i = 0; i < num; i++) {
             const PauliGroup& g = gs.g[i];
-            double res[GROUP_STRINGS];
-            rc = land(g.ticket, res, g.numStrings);
+            double res[LAND_VALUES];
+            rc = land(g.ticket, res, g.pairs ? 2 * g.nv : g.numStrings);
             if (rc != QA_OK) return rc;
+            if (g.pairs) {
+                const double* const c = res + g.nv;
+                const uint64_t own = g.numWork / ((uint64_t)reduceBlocks(g.numWork) * BLOCK) + 1;
+                bool all = true;
+                for (int t = 0; t < g.numStrings; t++) {
+                    const int mag = g.nv - 2 + (int)((g.odd >> t) & 1ull);
+                    all &= settled(res[t], c[t], res[mag] + c[mag], std::max(own, chains[i]), res[t]);
+                }
+                if (!all) {
+                    alone.push_back(Group{g.maskXY, first[i], g.numStrings});
+                    continue;
+                }
+            }
             for (int t = 0; t < g.numStrings; t++) {
                 const int64_t term = order[first[i] + t];
                 const double x = g.maskXY ? 2 * res[t] : res[t];

@@ -43,9 +43,7 @@ __device__ __forceinline__ void waveMerge(KB& acc) {
 // holding the result.  Lanes are paired at distances 32, 16, .. 1; while more
 // than one value is left, a pair splits them (each lane hands over one half
 // and merges the other), so a wave makes NV + 4 or so merges rather than
-// 6 NV (the sum of four groups of 5 strings over 25 qubits: 128 us instead of
-// 151, with half as many workgroups).  The pairing does not depend on NV, so
-// neither does a value's sum.
+// 6 NV.  The pairing does not depend on NV, so neither does a value's sum.
 template <int NV>
 __device__ void blockMerge(KB (&acc)[NV]) {
     constexpr int H = NV <= 1 ? 0 : NV <= 2 ? 1 : NV <= 4 ? 2 : NV <= 8 ? 3 : 4, P = 1 << H;

@@ -281,3 +281,65 @@ def test_full_state_diag_from_z_sum(api):
         api.destroyPauliStrSum(s)
         api.destroyFullStateDiagMatr(m)
         api.destroyQureg(q)
+
+
+def shared_read_terms(n, seed):
+    """(X, Y, Z) masks: groups of one to eight strings, with odd and even
+    numbers of Y, whose masks are XORs of others, low, high, or empty."""
+    rng = np.random.default_rng(seed)
+    top = 1 << (n - 1)
+    masks = [0b1, 0b11, top, top | 0b101, 1 << 7, (1 << 7) | 0b11, 0b110000, 0] + [int(m) for m in rng.integers(1, 1 << n, 3)]
+    terms = []
+    for i, m in enumerate(masks):
+        for _ in range(1 + (3 * i) % 8):
+            y = m & int(rng.integers(0, 1 << n))
+            terms.append((m & ~y, y, int(rng.integers(0, 1 << n)) & ~m))
+    return terms
+
+
+def state_for_shared_reads(kind, n):
+    rng = np.random.default_rng(n)
+    dim = 1 << n
+    if kind == "random":
+        a = rng.normal(size=dim) + 1j * rng.normal(size=dim)
+    elif kind == "real":  # strings with an odd number of Y have no terms but zeros
+        a = rng.normal(size=dim).astype(complex)
+    elif kind == "mirrored":  # a_n = a_{~n}: many sums are zero but for their rounding
+        h = rng.normal(size=dim // 2) + 1j * rng.normal(size=dim // 2)
+        a = np.concatenate([h, h[::-1]])
+    elif kind == "tie":  # sums halfway between two doubles, up to what cannot be seen
+        a = np.zeros(dim, complex)
+        a[[0, 1, 4, 5, 3, 128]] = [1, 1, 2.0 ** -27, 2.0 ** -27, 2.0 ** -60, 1]
+        return a
+    elif kind == "wide":  # magnitudes over 200 powers of two
+        a = rng.normal(size=dim) * 2.0 ** rng.integers(-100, 100, dim) * np.exp(2j * np.pi * rng.random(dim))
+    else:  # "infinite"
+        a = rng.normal(size=dim) + 1j * rng.normal(size=dim)
+        a[77] = np.inf
+        return a
+    return a / np.linalg.norm(a)
+
+
+@pytest.mark.parametrize("n,prec,kind", [(22, 2, "random"), (23, 2, "random"), (22, 1, "random"), (22, 2, "real"),
+                                         (22, 2, "mirrored"), (22, 2, "tie"), (22, 2, "wide"), (22, 2, "infinite")])
+def test_shared_reads_equal_single_string_reductions(api, n, prec, kind):
+    """From 22 qubits groups share reads of the state: a term's value is the
+    single string's, bit for bit, whatever the state."""
+    say(f"[gpu] pauli sum sharing reads n={n} prec={prec} {kind}")
+    terms = shared_read_terms(n, 17 + n)
+    nt = len(terms)
+    lib = api.gpu()
+    q = api.createCustomPrecisionQureg(n, 0, prec)
+    try:
+        api.set_amps(q, state_for_shared_reads(kind, n))
+        col = [(C.c_uint64 * nt)(*[t[i] for t in terms]) for i in range(3)]
+        coeffs = (C.c_double * (2 * nt))(*([1.0, 0.0] * nt))
+        vals, out, single = (C.c_double * (2 * nt))(), (C.c_double * 2)(), (C.c_double * 2)()
+        assert lib.qa_statevec_calcExpecPauliStrSum(C.c_void_p(q.gpuAmps), prec, n, C.c_int64(nt), *col, coeffs, vals,
+                                                    out) == 0
+        for t, (x, y, z) in enumerate(terms):
+            assert lib.qa_statevec_calcExpecPauliStr(C.c_void_p(q.gpuAmps), prec, n, C.c_uint64(x), C.c_uint64(y),
+                                                     C.c_uint64(z), single) == 0
+            assert np.array_equal(np.array(vals[2 * t:2 * t + 2]), np.array(single[:]), equal_nan=True), (t, x, y, z)
+    finally:
+        api.destroyQureg(q)
