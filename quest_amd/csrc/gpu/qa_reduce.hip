@@ -391,7 +391,7 @@ constexpr int GROUP_VALUES = GROUP_STRINGS + 2;  // of one partial, at most
 struct PauliGroup {
     uint64_t maskXY, topLow;  // topLow: the bits below the top X/Y bit
     uint64_t maskYZ[GROUP_STRINGS];
-    uint64_t odd;             // bit t: string t has an odd number of Y
+    uint64_t odd;             // bit t: maskXY and string t's maskYZ share an odd number of bits
     uint64_t numWork;
     int blocks, numStrings;
     int nv;                   // values of one partial: numStrings, or more
@@ -1276,7 +1276,9 @@ int expecStrings(const T* a, int nq, int64_t numTerms, const uint64_t* maskX, co
             for (int t = 0; t < x.num; t++) {
                 const int64_t term = order[x.first + t];
                 g.maskYZ[t] = maskY[term] | maskZ[term];
-                g.odd |= (uint64_t)(__builtin_popcountll(maskY[term]) & 1) << t;
+                // as many bits in both as there are Y; a single string may also
+                // have X and Z on one qubit, whose product it then is
+                g.odd |= (uint64_t)(__builtin_popcountll(x.mxy & g.maskYZ[t]) & 1) << t;
             }
             g.numWork = 1ull << (x.mxy ? nq - 1 : nq);
             g.blocks = reduceBlocks(g.numWork);

@@ -343,3 +343,24 @@ def test_shared_reads_equal_single_string_reductions(api, n, prec, kind):
             assert np.array_equal(np.array(vals[2 * t:2 * t + 2]), np.array(single[:]), equal_nan=True), (t, x, y, z)
     finally:
         api.destroyQureg(q)
+
+
+@pytest.mark.parametrize("masks", [(5, 2, 8), (5, 0, 4), (5, 0, 1), (3, 6, 0), (1, 2, 3), (7, 7, 7), (0, 0, 9)])
+def test_single_string_masks_may_overlap(api, masks):
+    """qa_statevec_calcExpecPauliStr sums conj(a_n) (-1)^|j & (Y|Z)| a_j over n,
+    j = n ^ (X|Y), times i^|Y|, whatever the three masks share."""
+    say(f"[gpu] single pauli string, masks {masks}")
+    n, (x, y, z) = 9, masks
+    amps = qc.random_state(n, 29)
+    q = api.createQureg(n)
+    out = (C.c_double * 2)()
+    try:
+        api.set_amps(q, amps)
+        assert api.gpu().qa_statevec_calcExpecPauliStr(C.c_void_p(q.gpuAmps), 2, n, C.c_uint64(x), C.c_uint64(y),
+                                                       C.c_uint64(z), out) == 0
+    finally:
+        api.destroyQureg(q)
+    j = np.arange(1 << n) ^ (x | y)
+    sign = np.array([1 - 2 * (bin(v & (y | z)).count("1") & 1) for v in j])
+    want = np.sum(sign * np.conj(amps) * amps[j]) * 1j ** bin(y).count("1")
+    assert abs(complex(out[0], out[1]) - want) <= 1e-14
