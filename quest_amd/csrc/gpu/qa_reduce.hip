@@ -193,8 +193,11 @@ __device__ __forceinline__ double norm2(cd a) { return a.re * a.re + a.im * a.im
 // both outcome probabilities of PQ qubits q0..q0+PQ-1 in one read of the
 // state: |a_n|^2 goes to o[b] when qubit q0 + b is 0 in n, to o[PQ + b]
 // when it is 1, so each outcome is the compensated sum of its own terms
-// (never a difference of two sums, which would lose a small probability)
-constexpr int PQ = 8;
+// (never a difference of two sums, which would lose a small probability).
+// Ten qubits a read: states of 33 to 40 qubits are read 4 times, states of
+// fewer than 10 once.
+constexpr int PQ = 10;
+static_assert(2 * PQ <= LAND_VALUES, "a read's values land in one slot");
 template <typename T>
 struct FProbsOfQubits {
     const T* a;

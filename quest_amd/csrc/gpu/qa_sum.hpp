@@ -46,8 +46,8 @@ __device__ __forceinline__ void waveMerge(KB& acc) {
 // 6 NV.  The pairing does not depend on NV, so neither does a value's sum.
 template <int NV>
 __device__ void blockMerge(KB (&acc)[NV]) {
-    constexpr int H = NV <= 1 ? 0 : NV <= 2 ? 1 : NV <= 4 ? 2 : NV <= 8 ? 3 : 4, P = 1 << H;
-    static_assert(NV <= 16, "values of one merge");
+    constexpr int H = NV <= 1 ? 0 : NV <= 2 ? 1 : NV <= 4 ? 2 : NV <= 8 ? 3 : NV <= 16 ? 4 : 5, P = 1 << H;
+    static_assert(NV <= 32, "values of one merge");
     __shared__ KB sh[BLOCK / 64][P];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     KB t[P];

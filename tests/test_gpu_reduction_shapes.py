@@ -123,3 +123,24 @@ def test_pauli_sums_sharing_reads(api, n, prec):
             par = par ^ (par >> sh)
         want = (1j ** bin(y).count("1")) * np.vdot(a[idx ^ (x | y)], (1 - 2 * (par & 1)) * a)
         assert abs(complex(vals[2 * t], vals[2 * t + 1]) - want) <= 1e-14, (t, bin(x | y))
+
+
+@pytest.mark.parametrize("n,prec", [(1, 2), (5, 1), (8, 2), (9, 2), (9, 1), (33, 1)])
+def test_every_qubit_probabilities_ten_at_a_time(api, n, prec):
+    """Below 10 qubits and above 32 (33: 64 GiB) a read serves up to ten
+    qubits; a product state has each qubit's probabilities in closed form.
+    The tolerance is the states' own: a gate rounds by a few units."""
+    print(f"[gpu] every-qubit probabilities ten at a time n={n} prec={prec}", flush=True)
+    angles = [0.2 + 0.08 * t for t in range(n)]
+    q = api.createCustomPrecisionQureg(n, 0, prec)
+    out = np.zeros(2 * n)
+    try:
+        api.initZeroState(q)
+        for t, x in enumerate(angles):
+            api.applyRotateY(q, t, x)
+        assert api.gpu().qa_statevec_calcProbsOfEveryQubit(C.c_void_p(q.gpuAmps), prec, n, out.ctypes.data_as(C.c_void_p)) == 0
+    finally:
+        api.destroyQureg(q)
+    tol = 4 * n * (2.0 ** -53 if prec == 2 else 2.0 ** -24)
+    assert np.max(np.abs(out[1::2] - np.sin(np.array(angles) / 2) ** 2)) <= tol
+    assert np.max(np.abs(out[0::2] - np.cos(np.array(angles) / 2) ** 2)) <= tol
