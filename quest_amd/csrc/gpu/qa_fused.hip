@@ -1106,10 +1106,17 @@ void fuse::clusterPass(const GOp* ops, size_t num, uint64_t avoid, std::vector<G
     }
 }
 
-bool fuse::layerable(const GOp* ops, size_t num) {
-    for (size_t i = 0; i < num; i++)
-        if (!signGate(ops[i]) && !(ops[i].kind == F_DENSE1 && !ops[i].cMask)) return false;
-    return true;
+bool fuse::layerable(const GOp* ops, size_t num, int prec) {
+    size_t matrices = 0, whole = 0;
+    for (size_t i = 0; i < num; i++) {
+        if (signGate(ops[i])) continue;
+        if (ops[i].kind != F_DENSE1 || ops[i].cMask) return false;
+        std::complex<double> factor, before, after;
+        double t;
+        matrices++;
+        whole += !splitUnitary(ops[i].f, prec, factor, before, after, t);
+    }
+    return 16 * whole <= matrices;
 }
 
 void fuse::layerPass(const GOp* ops, size_t num, uint64_t avoid, std::vector<GOp>& out) {

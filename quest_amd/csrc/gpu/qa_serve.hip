@@ -926,7 +926,7 @@ int qa_serveSubmit(void* engine, const qa_serveCircuit* c, int64_t* id) {
         setError("%s", err.c_str());
         return QA_ERR_ARG;
     }
-    r->layers = layerable(r->ops.data(), r->ops.size());
+    r->layers = layerable(r->ops.data(), r->ops.size(), E->prec);
     r->frame.prec = E->prec;
     r->left.resize(r->ops.size());
     for (size_t i = 0; i < r->left.size(); i++) r->left[i] = (uint32_t)i;

@@ -86,8 +86,13 @@ void mergePass(const GOp* ops, size_t num, uint64_t localMask, std::vector<GOp>&
 void clusterPass(const GOp* ops, size_t num, uint64_t avoid, std::vector<GOp>& out);
 
 // true when every op is an uncontrolled one-qubit matrix or a sign gate (a
-// diagonal of 1 and -1 under any controls), which layerPass takes
-bool layerable(const GOp* ops, size_t num);
+// diagonal of 1 and -1 under any controls), which layerPass takes, and at most
+// one in 16 matrices has to go as it is (X, Y and those near them, and what is
+// not unitary).  Such a matrix is an op of its own in a layer, where merged
+// passes multiply it into others: 16 requests of 22 qubits, 12 layers,
+// complex128 take 9.5 ms in layers of rotations, 10.7 with one X in 10, 12.3
+// with 3 in 10, 16.9 of X alone; merged 10.3-11.2 ms whatever the matrices.
+bool layerable(const GOp* ops, size_t num, int prec);
 
 // the ops of one such pass reordered in place of mergePass and clusterPass:
 // rounds on RB qubits each, in which all one-qubit matrices that nothing

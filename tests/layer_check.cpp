@@ -82,6 +82,44 @@ static bool oneMatrix(const cx (&m)[4], const char* what) {
     return false;
 }
 
+static bool layersOnly(const std::vector<GOp>& ops) {
+    for (const GOp& g : ops)
+        if (!(g.kind == F_DENSE1 && !g.cMask) && !(g.kind == F_DIAG1 && g.f[2] == -1.0)) return false;
+    return true;
+}
+
+// queues of rotations go as layers, those with many matrices that do not split
+// (here X) or with other gates do not
+static bool choices() {
+    for (int prec : {QA_FP64, QA_FP32})
+        for (int x : {0, 1, 2, 10, 32}) {
+            std::vector<GOp> ops;
+            for (int i = 0; i < 32; i++) {
+                GOp g;
+                g.kind = F_DENSE1;
+                g.t1 = i % 5;
+                const double th = i < x ? M_PI : 0.1 * i;
+                const double m[8] = {std::cos(th / 2), 0, 0, -std::sin(th / 2), 0, -std::sin(th / 2), std::cos(th / 2), 0};
+                std::memcpy(g.f, m, sizeof m);
+                ops.push_back(g);
+                GOp cz;
+                cz.kind = F_DIAG1;
+                cz.t1 = i % 5;
+                cz.cMask = cz.cVal = (1ull << cz.t1) | (1ull << ((i + 1) % 5));
+                cz.f[0] = 1;
+                cz.f[2] = -1;
+                ops.push_back(cz);
+            }
+            if (layerable(ops.data(), ops.size(), prec) != (x <= 2))
+                return std::printf("FAIL: layers chosen wrongly for %d of 32 matrices\n", x), false;
+            ops[40].cMask = 1ull << 7;
+            ops[40].cVal = 1ull << 7;
+            if (layerable(ops.data(), ops.size(), prec))
+                return std::printf("FAIL: layers chosen for a controlled matrix\n"), false;
+        }
+    return true;
+}
+
 static bool matrices() {
     const double h = std::sqrt(0.5), nan = std::nan("");
     const cx e = std::polar(1.0, 2.45), f = std::polar(1.0, -0.7);
@@ -117,7 +155,7 @@ static bool matrices() {
 }
 
 int main(int argc, char** argv) {
-    if (!matrices()) return 1;
+    if (!matrices() || !choices()) return 1;
     const int rounds = argc > 1 ? std::atoi(argv[1]) : 200;
     std::mt19937_64 rng(argc > 2 ? std::strtoull(argv[2], nullptr, 0) : 1);
     auto below = [&](int n) { return (int)(rng() % (uint64_t)n); };
@@ -184,7 +222,7 @@ int main(int argc, char** argv) {
             for (size_t i = 0; i < ops.size(); i++)
                 if (p < picked.size() && picked[p] == i) pass.push_back(ops[i]), p++;
                 else rest.push_back(ops[i]);
-            if (!layerable(pass.data(), pass.size())) return std::printf("FAIL: not layerable\n"), 1;
+            if (!layersOnly(pass)) return std::printf("FAIL: not layerable\n"), 1;
             layers.clear();
             layerPass(pass.data(), pass.size(), (1ull << low) - 1, layers);
             if (layers.size() != pass.size()) return std::printf("FAIL: %zu of %zu ops\n", layers.size(), pass.size()), 1;
