@@ -580,7 +580,7 @@ void frameGates(LayerFrame& frame, int numQubits, std::vector<GOp>& out) {
 }
 
 void emitGroups(const GOp* ops, size_t from, size_t to, Layout& L, int k, int low, std::vector<TOp>& prog,
-                GroupState& st, bool phases, bool signs = false, LayerFrame* frame = nullptr) {
+                GroupState& st, bool phases, LayerFrame* frame = nullptr) {
     size_t i = from;
     while (i < to) {
         if (isLdsOp(ops[i])) {
@@ -636,7 +636,7 @@ void emitGroups(const GOp* ops, size_t from, size_t to, Layout& L, int k, int lo
                     continue;
                 }
             }
-            if (signs && signGate(ops[i])) {
+            if (frame && signGate(ops[i])) {
                 TOp t;
                 std::memset(&t, 0, sizeof(t));
                 t.h.kind = F_SIGNS;
@@ -687,36 +687,10 @@ void emitGroups(const GOp* ops, size_t from, size_t to, Layout& L, int k, int lo
                 i += n;
                 continue;
             }
-            // with signs, 2-4 such gates on any different register bits
-            if (frame && ops[i].kind == F_DENSE1 && !ops[i].cMask) {
-                prog.push_back(toTile(takePhase(ops[i], *frame), L));
-                i++;
-                continue;
-            }
-            const GOp* on[RB] = {};
-            n = 0;
-            while (signs && i + n < j && ops[i + n].kind == F_DENSE1 && !ops[i + n].cMask) {
-                const GOp*& at = on[L.regOf[L.slotOf[ops[i + n].t1]]];
-                if (at) break;
-                at = &ops[i + n++];
-            }
-            if (n >= 2) {
-                TOp t;
-                std::memset(&t, 0, sizeof(t));
-                t.h.kind = F_DENSE1S;
-                int at = 0;
-                for (int b = 0; b < RB; b++) {
-                    if (!on[b]) continue;
-                    t.h.rb1 |= 1 << b;
-                    std::memcpy(at ? (void*)(t.fx + 8 * (at - 1)) : (void*)t.b, on[b]->f, 8 * sizeof(double));
-                    at++;
-                }
-                prog.push_back(t);
-                i += n;
-            } else {
-                prog.push_back(toTile(ops[i], L));
-                i++;
-            }
+            // (with a frame, a matrix here is one that layerOp leaves)
+            const bool matrix = frame && ops[i].kind == F_DENSE1 && !ops[i].cMask;
+            prog.push_back(toTile(matrix ? takePhase(ops[i], *frame) : ops[i], L));
+            i++;
         }
     }
 }
@@ -1208,7 +1182,7 @@ void fuse::layerPass(const GOp* ops, size_t num, uint64_t avoid, std::vector<GOp
 }
 
 void fuse::planPass(const GOp* ops, size_t num, int numQubits, uint64_t localMask, int lowQubits, TileArgs& a,
-                    std::vector<TOp>& prog, bool phases, bool signs, LayerFrame* frame) {
+                    std::vector<TOp>& prog, bool phases, LayerFrame* frame) {
     Layout L;
     passShape(numQubits, localMask, a, L);
     const int k = a.k;
@@ -1216,7 +1190,7 @@ void fuse::planPass(const GOp* ops, size_t num, int numQubits, uint64_t localMas
     const uint32_t lowSlots = (1u << low) - 1u;
     const size_t start = prog.size();
     GroupState st;
-    emitGroups(ops, 0, num, L, k, low, prog, st, phases, signs, frame);
+    emitGroups(ops, 0, num, L, k, low, prog, st, phases, frame);
     if (frame && frame->finish) {
         std::vector<GOp> rest;
         frameGates(*frame, numQubits, rest);

@@ -472,8 +472,7 @@ bool launchStep(Engine& E, StepBuf& sb, std::string& err) {
                 clusterPass(merged.data(), merged.size(), (1ull << low) - 1ull, pass);
             }
             r->frame.finish = r->left.empty();
-            planPass(pass.data(), pass.size(), r->n, L, E.lowQ, pd.a, prog, true, r->layers,
-                     r->layers ? &r->frame : nullptr);
+            planPass(pass.data(), pass.size(), r->n, L, E.lowQ, pd.a, prog, true, r->layers ? &r->frame : nullptr);
             setLdsOffsets(prog.data() + pd.opsOffset, prog.size() - pd.opsOffset, pd.a, E.prec);
             r->firstPass = false;
             byK[pd.a.k].push_back(pd);

@@ -97,9 +97,9 @@ bool layerable(const GOp* ops, size_t num, int prec);
 // the ops of one such pass reordered in place of mergePass and clusterPass:
 // rounds on RB qubits each, in which all one-qubit matrices that nothing
 // earlier holds back go together, then all the sign gates that some further
-// matrix of the round waits for, and so on.  The runs become DENSE1N /
-// DENSE1S and SIGNS ops (planPass with signs), so that a pass is little more
-// than its matrices' arithmetic.
+// matrix of the round waits for, and so on.  The runs become LAYER
+// and SIGNS ops (planPass with a frame), so that a pass is little more than its
+// matrices' arithmetic.
 void layerPass(const GOp* ops, size_t num, uint64_t avoid, std::vector<GOp>& out);
 
 // the program of one pass applying ops[0..num) (dense targets all inside
@@ -107,11 +107,11 @@ void layerPass(const GOp* ops, size_t num, uint64_t avoid, std::vector<GOp>& out
 // but the LDS offsets and appends the ops, with their GROUP ops, to `prog`;
 // with `phases`, runs of diagonal gates become PHASES ops (their factors are
 // then multiplied before they reach the amplitudes, which changes rounding);
-// with `signs` (the serving engine's programs), runs of sign gates become
-// SIGNS ops, and with a frame too, layers of one-qubit unitaries LAYER ops
+// with a frame (the serving engine's programs of layers), runs of sign gates
+// become SIGNS ops and layers of one-qubit unitaries LAYER ops
 struct LayerFrame;
 void planPass(const GOp* ops, size_t num, int numQubits, uint64_t localMask, int lowQubits, TileArgs& a,
-              std::vector<TOp>& prog, bool phases = false, bool signs = false, LayerFrame* frame = nullptr);
+              std::vector<TOp>& prog, bool phases = false, LayerFrame* frame = nullptr);
 
 // The phases diag(1, f[q]) that a state still lacks on each qubit: LAYER ops
 // leave a unitary's last phase to the next one on its qubit, over passes too.

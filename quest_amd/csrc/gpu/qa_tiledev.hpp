@@ -34,7 +34,7 @@ constexpr int RB = 4;        // register slots per group
 constexpr int RA = 1 << RB;  // amplitudes per thread
 enum {
     F_GROUP = 100, F_BLOCK = 101, F_DENSE1N = 102, F_PAULI_LDS = 103, F_PHASES = 104, F_DENSE_LDS = 105,
-    F_SIGNS = 106, F_DENSE1S = 107, F_LAYER = 108
+    F_SIGNS = 106, F_LAYER = 107
 };
 constexpr int BQ = 5;  // qubits of an MFMA block (32 x 32 complex)
 
@@ -857,19 +857,6 @@ __device__ __forceinline__ void applyOp(ct<T>* r, const TOp* __restrict__ op, co
         case F_SIGNS:
             if constexpr (SV)
                 applySigns<T>(r, uniformAt<SignTerm>(op->b), h.rb2, h.rb1, jb, base);
-            break;
-        case F_DENSE1S: if constexpr (SV) {
-            // uncontrolled one-qubit matrices on the register bits set in
-            // rb1, in ascending order: the first in the body, the rest in fx
-            const double* fx = op->fx - 8;
-            if (h.rb1 & 1) regDense1<T, 0, false>(r, h, m2At<T>(f));
-            if (h.rb1 & 2) regDense1<T, 1, false>(r, h, m2At<T>((h.rb1 & 1) ? fx + 8 : f));
-            if (h.rb1 & 4) {
-                const int k = __popc((uint32_t)h.rb1 & 3u);
-                regDense1<T, 2, false>(r, h, m2At<T>(k ? fx + 8 * k : f));
-            }
-            if (h.rb1 & 8) regDense1<T, 3, false>(r, h, m2At<T>(fx + 8 * __popc((uint32_t)h.rb1 & 7u)));
-        }
             break;
         case F_DEPOL1:
             if constexpr (!SV) {

@@ -1,9 +1,8 @@
 // Plans random passes of one-qubit matrices and sign gates with the
 // library's layerPass and planPass and applies the planned programs -- op by
-// op, with a restatement of LAYER, DENSE1, DENSE1N, DENSE1S, SIGNS, PHASES,
-// GROUP and DIAG1 over whole states -- against the gates in queue order.  Every
-// other queue is planned with a frame (LAYER ops); its matrices are unitaries
-// of every kind, the ones that a layer leaves out among them.
+// op, with a restatement of LAYER, DENSE1, SIGNS, PHASES, GROUP and DIAG1 over
+// whole states -- against the gates in queue order.  The matrices are unitaries
+// of every kind and others, the ones that a layer leaves out among them.
 #include <cmath>
 #include <complex>
 #include <cstdio>
@@ -40,7 +39,7 @@ static bool oneMatrix(const cx (&m)[4], const char* what) {
     frame.finish = true;
     TileArgs a;
     std::vector<TOp> prog;
-    planPass(&g, 1, n, (1ull << n) - 1, 0, a, prog, true, true, &frame);
+    planPass(&g, 1, n, (1ull << n) - 1, 0, a, prog, true, &frame);
     // each column of the product of the program's ops on the one qubit
     double worst = 0;
     for (int col = 0; col < 2; col++) {
@@ -144,7 +143,7 @@ static bool matrices() {
         for (int i = 0; i < 4; i++) g.f[2 * i] = m[i].real(), g.f[2 * i + 1] = m[i].imag();
         TileArgs a;
         std::vector<TOp> prog;
-        planPass(&g, 1, 4, 15, 0, a, prog, true, true, &frame);
+        planPass(&g, 1, 4, 15, 0, a, prog, true, &frame);
         // a matrix that is no unitary goes as it is
         bool kept = false;
         for (const TOp& t : prog)
@@ -160,10 +159,9 @@ int main(int argc, char** argv) {
     std::mt19937_64 rng(argc > 2 ? std::strtoull(argv[2], nullptr, 0) : 1);
     auto below = [&](int n) { return (int)(rng() % (uint64_t)n); };
     auto uniform = [&] { return 2.0 * (double)(rng() >> 11) / 9007199254740992.0 - 1; };
-    long signOps = 0, subsetOps = 0, layerOps = 0;
+    long signOps = 0, layerOps = 0;
     for (int round = 0; round < rounds; round++) {
         const int n = 4 + below(6), kMax = 4 + below(n - 3), low = below(std::min(kMax, 3) + 1);
-        const bool framed = round & 1;
         LayerFrame frame;
         std::vector<GOp> ops;
         const int num = 1 + below(60);
@@ -173,7 +171,7 @@ int main(int argc, char** argv) {
                 g.kind = F_DENSE1;
                 g.t1 = below(n);
                 for (int k = 0; k < 8; k++) g.f[k] = uniform();
-                if (framed && below(8)) {
+                if (below(8)) {
                     // e^{ia} [[c, -s e^{il}], [s e^{ip}, c e^{i(l+p)}]]: any angle, or a (nearly) diagonal or
                     // antidiagonal one
                     const double special[] = {0, 1e-12, 1e-7, M_PI / 2, M_PI / 2 - 1e-5, M_PI, 0.78539816339744828,
@@ -229,7 +227,7 @@ int main(int argc, char** argv) {
             TileArgs a;
             std::vector<TOp> prog;
             frame.finish = rest.empty();
-            planPass(layers.data(), layers.size(), n, L, low, a, prog, true, true, framed ? &frame : nullptr);
+            planPass(layers.data(), layers.size(), n, L, low, a, prog, true, &frame);
             int slots[RB] = {0, 0, 0, 0};
             for (const TOp& t : prog) {
                 auto qubit = [&](int b) { return a.localPos[slots[b]]; };
@@ -237,19 +235,6 @@ int main(int argc, char** argv) {
                 switch (t.h.kind) {
                     case F_GROUP: std::memcpy(slots, t.b, sizeof(slots)); break;
                     case F_DENSE1: dense1(got, qubit(t.h.rb1), b); break;
-                    case F_DENSE1N:
-                        for (int m = 0; m < t.h.rb2; m++) dense1(got, qubit(m), m ? t.fx + 8 * (m - 1) : b);
-                        break;
-                    case F_DENSE1S: {
-                        int m = 0;
-                        for (int r = 0; r < RB; r++)
-                            if ((t.h.rb1 >> r) & 1) {
-                                dense1(got, qubit(r), m ? t.fx + 8 * (m - 1) : b);
-                                m++;
-                            }
-                        subsetOps++;
-                        break;
-                    }
                     case F_SIGNS: case F_LAYER: case F_PHASES: case F_DIAG1: {
                         const LayerBody<double>& body = *reinterpret_cast<const LayerBody<double>*>(t.b);
                         const bool layer = t.h.kind == F_LAYER;
@@ -309,6 +294,6 @@ int main(int argc, char** argv) {
             return 1;
         }
     }
-    std::printf("ok: %d queues, %ld sign ops, %ld subset ops, %ld layer ops\n", rounds, signOps, subsetOps, layerOps);
-    return signOps && subsetOps && layerOps ? 0 : 1;
+    std::printf("ok: %d queues, %ld sign ops, %ld layer ops\n", rounds, signOps, layerOps);
+    return signOps && layerOps ? 0 : 1;
 }
