@@ -455,36 +455,40 @@ SignTerm signTerm(const GOp& g, const Layout& L) {
     return t;
 }
 
-// m as factor * diag(1, after) [[1, -t], [t, 1]] diag(1, before), `factor`
-// being its first element and the phases of modulus 1; false (a DENSE1 op is
-// then made of it) when it is not unitary, or when its diagonal is so small
-// that the scaled amplitudes would leave the storage's middle range.  The
-// element b is not used but follows from the others, so "unitary" is to a few
-// units of FP64 in a complex128 state (rotations, their products and Haar
-// matrices are within 1 to 3 of 2^-52) and well below a unit of the storage in
-// a complex64 one; a NaN in any element fails the comparisons.
-bool splitUnitary(const double* m, int prec, std::complex<double>& factor, std::complex<double>& before,
+// Whether a layer takes the matrix m (splitUnitary): not when it is not
+// unitary, nor when its diagonal is so small that the scaled amplitudes would
+// leave the storage's middle range.  The element b is not used but follows from
+// the others, so "unitary" is to a few units of FP64 in a complex128 state
+// (rotations, their products and Haar matrices are within 1 to 3 of 2^-52) and
+// well below a unit of the storage in a complex64 one; a NaN in any element
+// fails the comparisons.
+bool splits(const double* m, int prec) {
+    const double eps = prec == QA_FP64 ? 0x1p-50 : 1e-13;
+    const double na = m[0] * m[0] + m[1] * m[1], nb = m[2] * m[2] + m[3] * m[3];
+    const double nc = m[4] * m[4] + m[5] * m[5], nd = m[6] * m[6] + m[7] * m[7];
+    // conj(a) b + conj(c) d
+    const double re = m[0] * m[2] + m[1] * m[3] + m[4] * m[6] + m[5] * m[7];
+    const double im = m[0] * m[3] - m[1] * m[2] + m[4] * m[7] - m[5] * m[6];
+    return std::fabs(na + nc - 1) <= eps && std::fabs(nb + nd - 1) <= eps && re * re + im * im <= eps * eps &&
+           na >= 0x1p-16;
+}
+
+// m, one that splits, as factor * diag(1, after) [[1, -t], [t, 1]]
+// diag(1, before), `factor` being its first element and the phases of modulus 1
+void splitUnitary(const double* m, std::complex<double>& factor, std::complex<double>& before,
                   std::complex<double>& after, double& t) {
     typedef std::complex<double> cx;
-    const cx a(m[0], m[1]), b(m[2], m[3]), c(m[4], m[5]), d(m[6], m[7]);
-    const double eps = prec == QA_FP64 ? 0x1p-50 : 1e-13;
-    if (!(std::abs(std::norm(a) + std::norm(c) - 1) <= eps && std::abs(std::norm(b) + std::norm(d) - 1) <= eps &&
-          std::abs(std::conj(a) * b + std::conj(c) * d) <= eps))
-        return false;
-    const double co = std::abs(a);
-    if (co < 1.0 / 256) return false;
-    const cx e = a / co;
+    const cx a(m[0], m[1]), c(m[4], m[5]), d(m[6], m[7]);
+    auto unit = [](const cx& z) { return z / std::sqrt(std::norm(z)); };
+    const cx e = unit(a);
     factor = a;
-    t = std::abs(c) / co;
+    t = std::abs(c) / std::sqrt(std::norm(a));
     // `after` from c and `before` from d, so that an error of after's phase
     // (c may be small) is not in d.  A c among the subnormals has few bits, and
     // a quotient of two of them fewer: its phase is taken from c scaled up.
     const cx up = std::norm(c) < 0x1p-900 ? c * 0x1p+900 : c;
-    after = up == cx(0) ? cx(1) : up / (e * std::abs(up));
-    after /= std::abs(after);
-    before = d / (e * after);
-    before /= std::abs(before);
-    return true;
+    after = up == cx(0) ? cx(1) : unit(unit(up) * std::conj(e));
+    before = unit(d * std::conj(e * after));
 }
 
 template <typename T>
@@ -522,8 +526,9 @@ size_t layerOp(const GOp* ops, size_t num, const Layout& L, LayerFrame& frame, s
     for (; n < num && ops[n].kind == F_DENSE1 && !ops[n].cMask; n++) {
         const int q = ops[n].t1, b = L.regOf[L.slotOf[q]];
         if ((mask >> b) & 1) break;
+        if (!splits(ops[n].f, frame.prec)) break;
         cx factor;
-        if (!splitUnitary(ops[n].f, frame.prec, factor, before[b], after[b], rot[b])) break;
+        splitUnitary(ops[n].f, factor, before[b], after[b], rot[b]);
         scale *= factor;
         before[b] *= frame.f[q];
         qubit[b] = q;
@@ -1085,10 +1090,8 @@ bool fuse::layerable(const GOp* ops, size_t num, int prec) {
     for (size_t i = 0; i < num; i++) {
         if (signGate(ops[i])) continue;
         if (ops[i].kind != F_DENSE1 || ops[i].cMask) return false;
-        std::complex<double> factor, before, after;
-        double t;
         matrices++;
-        whole += !splitUnitary(ops[i].f, prec, factor, before, after, t);
+        whole += !splits(ops[i].f, prec);
     }
     return 16 * whole <= matrices;
 }
