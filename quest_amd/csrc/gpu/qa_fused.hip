@@ -713,11 +713,18 @@ uint64_t supportMask(const GOp& g) {
 }
 
 // g applied to a vector of 2^nq amplitudes whose bit b is global qubit q[b]
-// (every qubit of g is one of them), in FP64, with the same semantics as
+// (every qubit of g is one of them), in precision R, with the same semantics as
 // the single-gate kernels; false, with v untouched, for a kind whose action is
-// not known on the host (a DENSEN matrix is in device memory)
-bool applySmall(const GOp& g, const int* q, int nq, std::complex<double>* v) {
-    typedef std::complex<double> cx;
+// not known on the host (a DENSEN matrix is in device memory).  The vectors are
+// unit vectors that some gates have been applied to, mostly zeros: pairs and
+// products of zeros are left out.
+template <typename R>
+bool applySmall(const GOp& g, const int* q, int nq, std::complex<R>* v) {
+    typedef std::complex<R> cx;
+    const cx zero(0);
+    auto mul = [](const cx& x, const cx& y) {
+        return cx(x.real() * y.real() - x.imag() * y.imag(), x.real() * y.imag() + x.imag() * y.real());
+    };
     auto loc = [&](uint64_t m) {
         uint32_t r = 0;
         for (int b = 0; b < nq; b++)
@@ -731,15 +738,16 @@ bool applySmall(const GOp& g, const int* q, int nq, std::complex<double>* v) {
     };
     const uint32_t cm = loc(g.cMask), cv = loc(g.cVal);
     const int D = 1 << nq;
-    auto fc = [&](int i) { return cx(g.f[2 * i], g.f[2 * i + 1]); };
+    auto fc = [&](int i) { return cx((R)g.f[2 * i], (R)g.f[2 * i + 1]); };
     switch (g.kind) {
         case F_DENSE1: {
             const uint32_t t = 1u << bitOf(g.t1);
             for (int j = 0; j < D; j++) {
                 if ((j & t) || (j & cm) != cv) continue;
                 const cx a0 = v[j], a1 = v[j | t];
-                v[j] = fc(0) * a0 + fc(1) * a1;
-                v[j | t] = fc(2) * a0 + fc(3) * a1;
+                if (a0 == zero && a1 == zero) continue;
+                v[j] = mul(fc(0), a0) + mul(fc(1), a1);
+                v[j | t] = mul(fc(2), a0) + mul(fc(3), a1);
             }
             break;
         }
@@ -754,8 +762,8 @@ bool applySmall(const GOp& g, const int* q, int nq, std::complex<double>* v) {
                 for (int b = 0; b < nv; b++) w |= ((j >> vb[b]) & 1) << b;
                 const double* m = g.f + 8 * w;
                 const cx a0 = v[j], a1 = v[j | t];
-                v[j] = cx(m[0], m[1]) * a0 + cx(m[2], m[3]) * a1;
-                v[j | t] = cx(m[4], m[5]) * a0 + cx(m[6], m[7]) * a1;
+                v[j] = mul(cx(m[0], m[1]), a0) + mul(cx(m[2], m[3]), a1);
+                v[j | t] = mul(cx(m[4], m[5]), a0) + mul(cx(m[6], m[7]), a1);
             }
             break;
         }
@@ -766,9 +774,9 @@ bool applySmall(const GOp& g, const int* q, int nq, std::complex<double>* v) {
                 if ((j & (t1 | t2)) || (j & cm) != cv) continue;
                 cx x[4], y[4];
                 for (int c = 0; c < 4; c++) x[c] = v[j | off[c]];
-                for (int r = 0; r < 4; r++) {
-                    y[r] = 0;
-                    for (int c = 0; c < 4; c++) y[r] += fc(4 * r + c) * x[c];
+                for (int c = 0; c < 4; c++) {
+                    if (x[c] == zero) continue;
+                    for (int r = 0; r < 4; r++) y[r] += mul(fc(4 * r + c), x[c]);
                 }
                 for (int r = 0; r < 4; r++) v[j | off[r]] = y[r];
             }
@@ -777,13 +785,13 @@ bool applySmall(const GOp& g, const int* q, int nq, std::complex<double>* v) {
         case F_DIAG1: {
             const uint32_t t = 1u << bitOf(g.t1);
             for (int j = 0; j < D; j++)
-                if ((j & cm) == cv) v[j] *= (j & t) ? fc(1) : fc(0);
+                if ((j & cm) == cv && v[j] != zero) v[j] = mul((j & t) ? fc(1) : fc(0), v[j]);
             break;
         }
         case F_PARITY: {
             const uint32_t m = loc(g.m1);
             for (int j = 0; j < D; j++)
-                if ((j & cm) == cv) v[j] *= (__builtin_popcount(j & m) & 1) ? fc(1) : fc(0);
+                if ((j & cm) == cv && v[j] != zero) v[j] = mul((__builtin_popcount(j & m) & 1) ? fc(1) : fc(0), v[j]);
             break;
         }
         case F_PAULI: {
@@ -792,11 +800,12 @@ bool applySmall(const GOp& g, const int* q, int nq, std::complex<double>* v) {
             for (int j = 0; j < D; j++) {
                 if ((j & top) || (j & cm) != cv) continue;
                 const int kk = j ^ mxy;
-                const double sA = (__builtin_popcount(j & myz) & 1) ? -1 : 1;
-                const double sB = (__builtin_popcount(kk & myz) & 1) ? -1 : 1;
                 const cx va = v[j], vb = v[kk];
-                v[j] = fc(0) * va + fc(1) * sB * vb;
-                v[kk] = fc(0) * vb + fc(1) * sA * va;
+                if (va == zero && vb == zero) continue;
+                const cx pA = (__builtin_popcount(j & myz) & 1) ? -fc(1) : fc(1);
+                const cx pB = (__builtin_popcount(kk & myz) & 1) ? -fc(1) : fc(1);
+                v[j] = mul(fc(0), va) + mul(pB, vb);
+                v[kk] = mul(fc(0), vb) + mul(pA, va);
             }
             break;
         }
@@ -810,7 +819,7 @@ bool applySmall(const GOp& g, const int* q, int nq, std::complex<double>* v) {
         }
         case F_DEPOL1: {
             const uint32_t k1 = 1u << bitOf(g.t1), k2 = 1u << bitOf(g.t2);
-            const double c1 = g.f[0], c2 = g.f[1], c3 = g.f[2];
+            const R c1 = g.f[0], c2 = g.f[1], c3 = g.f[2];
             for (int j = 0; j < D; j++) {
                 if (j & (k1 | k2)) continue;
                 const cx a00 = v[j], a11 = v[j | k1 | k2];
@@ -824,18 +833,18 @@ bool applySmall(const GOp& g, const int* q, int nq, std::complex<double>* v) {
         case F_DEPH1: {
             const uint32_t k1 = 1u << bitOf(g.t1), k2 = 1u << bitOf(g.t2);
             for (int j = 0; j < D; j++)
-                if (((j & k1) != 0) != ((j & k2) != 0)) v[j] *= g.f[0];
+                if (((j & k1) != 0) != ((j & k2) != 0)) v[j] *= (R)g.f[0];
             break;
         }
         case F_DEPH2: {
             const uint32_t a = loc(g.m1), b = loc(g.m2);
             for (int j = 0; j < D; j++)
-                if ((__builtin_popcount(j & a) | __builtin_popcount(j & b)) & 1) v[j] *= g.f[0];
+                if ((__builtin_popcount(j & a) | __builtin_popcount(j & b)) & 1) v[j] *= (R)g.f[0];
             break;
         }
         case F_DAMP1: case F_PAULIS1: {
             const uint32_t k1 = 1u << bitOf(g.t1), k2 = 1u << bitOf(g.t2);
-            const double* f = g.f;
+            const R f[4] = {(R)g.f[0], (R)g.f[1], (R)g.f[2], (R)g.f[3]};
             for (int j = 0; j < D; j++) {
                 if (j & (k1 | k2)) continue;
                 cx &a00 = v[j], &a01 = v[j | k1], &a10 = v[j | k2], &a11 = v[j | k1 | k2];
@@ -860,11 +869,11 @@ bool applySmall(const GOp& g, const int* q, int nq, std::complex<double>* v) {
             const uint32_t dA = a | braA, dB = b | braB;
             for (int j = 0; j < D; j++) {
                 if (j & (dA | dB)) continue;
-                const cx share = g.f[1] * (v[j] + v[j | dA] + v[j | dB] + v[j | dA | dB]);
+                const cx share = (R)g.f[1] * (v[j] + v[j | dA] + v[j | dB] + v[j | dA | dB]);
                 for (uint32_t w = 0; w < 16; w++) {
                     const bool ka = w & 1, kb = w & 2, ba = w & 4, bb = w & 8;
                     cx& x = v[j | (ka ? a : 0) | (kb ? b : 0) | (ba ? braA : 0) | (bb ? braB : 0)];
-                    x = ka == ba && kb == bb ? g.f[0] * x + share : g.f[2] * x;
+                    x = ka == ba && kb == bb ? (R)g.f[0] * x + share : (R)g.f[2] * x;
                 }
             }
             break;
@@ -929,9 +938,30 @@ bool mergeable(const GOp& g) {
 }
 bool diagonalOp(const GOp& g) { return g.kind == F_DIAG1 || g.kind == F_PARITY || g.kind == F_DEPH1; }
 
+// the matrix (row-major, nq <= 3 qubits q) of ops[members] in order, worked out
+// in precision R: its columns are the gates applied to the unit vectors, all at
+// once, as a vector that has a bit for each column bit beside the qubits
+template <typename R>
+void productOf(const GOp* ops, const std::vector<uint32_t>& members, const int* q, int nq, std::complex<double>* M) {
+    const int D = 1 << nq;
+    int bits[6];
+    for (int b = 0; b < nq; b++) {
+        bits[b] = q[b];
+        bits[nq + b] = 63;  // no qubit
+    }
+    std::complex<R> v[64] = {};
+    for (int c = 0; c < D; c++) v[c | c << nq] = 1;
+    for (uint32_t m : members) (void)applySmall(ops[m], bits, 2 * nq, v);  // knows every mergeable kind
+    for (int r = 0; r < D; r++)
+        for (int c = 0; c < D; c++) {
+            const std::complex<R>& e = v[r | c << nq];
+            M[r * D + c] = std::complex<double>((double)e.real(), (double)e.imag());
+        }
+}
+
 }  // namespace fuse
 
-void fuse::mergePass(const GOp* ops, size_t num, uint64_t localMask, std::vector<GOp>& out) {
+void fuse::mergePass(const GOp* ops, size_t num, uint64_t localMask, std::vector<GOp>& out, int prec) {
     struct Block {
         uint64_t qubits;                // local qubits
         uint64_t variants;              // non-local qubits (members are diagonal in them)
@@ -962,12 +992,8 @@ void fuse::mergePass(const GOp* ops, size_t num, uint64_t localMask, std::vector
             if ((b.variants >> x) & 1ull) q[nq++] = x;
         const int D = 1 << nq, DL = 1 << nl;
         std::complex<double> M[64];
-        for (int c = 0; c < D; c++) {
-            std::complex<double> v[8] = {};
-            v[c] = 1.0;
-            for (uint32_t m : b.members) (void)applySmall(ops[m], q, nq, v);  // knows every mergeable kind
-            for (int r = 0; r < D; r++) M[r * D + c] = v[r];
-        }
+        if (prec == QA_FP64) productOf<long double>(ops, b.members, q, nq, M);
+        else productOf<double>(ops, b.members, q, nq, M);
         GOp g;
         g.t1 = q[0];
         if (nq == nl) {
@@ -1773,7 +1799,7 @@ int flushQueue(void* amps, Queue& qu) {
         takePicked(ops.data(), left, picked, pass);
         const size_t numGates = pass.size();
         merged.clear();
-        mergePass(pass.data(), pass.size(), L, merged);
+        mergePass(pass.data(), pass.size(), L, merged, qu.prec);
         pass.clear();
         clusterPass(merged.data(), merged.size(), (1ull << low) - 1ull, pass);
         rc = launchPass(amps, qu, pass, 0, pass.size(), L, numGates);

@@ -814,9 +814,77 @@ static int blocksMain(int cases, uint64_t seed0) {
     return numBlocks && numLds && numDepol ? 0 : 1;
 }
 
+// ---- merged matrices ----------------------------------------------------------
+
+// runs of gates on two qubits: the one matrix that they become is their product,
+// each element rounded once
+static int roundingMain(int cases, uint64_t seed0) {
+    typedef std::complex<long double> lx;
+    double worst = 0;
+    for (int c = 0; c < cases; c++) {
+        Rng r(seed0 * 15485863ull + (uint64_t)c);
+        const int n = 6, qa = 1 + r.below(2), qb = 3 + r.below(2);
+        std::vector<GOp> queue, merged;
+        std::vector<lx> want(16, lx(0));
+        for (int i = 0; i < 4; i++) want[5 * i] = 1;
+        for (int i = 3 + r.below(10); i > 0; i--) {
+            GOp g;
+            lx m[16] = {};
+            if (r.below(2)) {
+                g.kind = F_DENSE1;
+                const int b = r.below(2);
+                g.t1 = b ? qb : qa;
+                randomUnitary2(r, g.f);
+                for (int row = 0; row < 4; row++)
+                    for (int e = 0; e < 2; e++) {
+                        const int col = (row & ~(1 << b)) | e << b, k = 2 * ((row >> b) & 1) + e;
+                        m[4 * row + col] = lx(g.f[2 * k], g.f[2 * k + 1]);
+                    }
+            } else {
+                // exp(i t XX) or, with signs, YY
+                g.kind = F_PAULI;
+                g.m1 = (1ull << qa) | (1ull << qb);
+                g.m2 = r.below(2) ? g.m1 : 0;
+                const double t = r.unit();
+                g.f[0] = std::cos(t);
+                g.f[3] = std::sin(t);
+                for (int row = 0; row < 4; row++) {
+                    const double s = g.m2 && (parity((uint64_t)row) != 0) ? -1 : 1;
+                    m[4 * row + row] = g.f[0];
+                    m[4 * row + (row ^ 3)] = lx(0, s * g.f[3]);
+                }
+            }
+            std::vector<lx> next(16, lx(0));
+            for (int row = 0; row < 4; row++)
+                for (int col = 0; col < 4; col++)
+                    for (int k = 0; k < 4; k++) next[4 * row + col] += m[4 * row + k] * want[4 * k + col];
+            want = next;
+            queue.push_back(g);
+        }
+        mergePass(queue.data(), queue.size(), (1ull << n) - 1ull, merged);
+        bool dense = merged.size() == 1 && merged[0].kind == F_DENSE2;
+        if (!dense) {  // gates on one of the qubits only
+            if (merged.size() > 2) return std::printf("case %d: %zu ops\n", c, merged.size()), 1;
+            continue;
+        }
+        for (int i = 0; i < 16; i++)
+            for (int part = 0; part < 2; part++) {
+                const long double w = part ? want[i].imag() : want[i].real();
+                const long double off = std::fabs((long double)merged[0].f[2 * i + part] - w);
+                // half a unit of the element, and what extended precision leaves
+                if (!(off <= 0x1p-53L * std::fabs(w) + 0x1p-58L))
+                    return std::printf("case %d: element %d off by %.3Le of %.3Le\n", c, i, off, w), 1;
+                worst = std::max(worst, (double)off);
+            }
+    }
+    std::printf("rounding check: %d cases agree (worst %.2e)\n", cases, worst);
+    return 0;
+}
+
 int main(int argc, char** argv) {
     const int cases = argc > 1 ? std::atoi(argv[1]) : 200;
     const uint64_t seed0 = argc > 2 ? std::strtoull(argv[2], nullptr, 10) : 1;
+    if (argc > 3 && std::string(argv[3]) == "rounding") return roundingMain(cases, seed0);
     if (argc > 3 && std::string(argv[3]) == "blocks") return blocksMain(cases, seed0);
     if (argc > 3 && std::string(argv[3]) == "span") return spanMain(cases, seed0);
     JitCheck jit;
