@@ -1727,20 +1727,28 @@ int flushQueue(void* amps, Queue& qu) {
     int rc = QA_OK;
     SpanArgs span;
     std::vector<SpanOp>& spanProg = g_spanProg;
-    // a span pass instead of the next tile pass when it takes more than one
-    // and a half times the gates, which is what one costs beside the other:
-    // at 21 qubits (double) a span pass of a few gadgets takes 45 us and a
-    // tile pass 30.  A Trotter step there took 342 us with the line at "more
-    // gates" and takes 298 with this one, at 25 qubits 1957 and 1698; a line
-    // at twice the gates measures the same, and no span passes at all cost
-    // layers with random gadgets 8190 us instead of 6620 (25 qubits) and 547
-    // instead of 396 (22 qubits, single).  (force: the front gadget fits no
-    // tile, so a span pass takes it alone if need be)
+    // a span pass instead of the next tile pass when it takes more gates for
+    // its cost.  Tile passes cost the state's traffic, whatever they hold
+    // (gadgets on the same qubits merge); a span pass of r gadgets costs as
+    // much up to 8 of them and 0.4 + 0.07 r times that beyond (26 qubits
+    // complex128: tile pass 0.50 ms, span pass of 8 0.49, of 16 0.74, of 30
+    // 1.15; alike from 20 to 28 qubits and in complex64).  Against taking the
+    // one with more gates, us a step:
+    //   complex128                20        22        24        26         28
+    //   nearest-neighbour XX, YY, ZZ
+    //                             161/153   226/228   491/494   2191/2014  7527/7611
+    //   XZX and YZY of neighbours 111/119   215/185   543/454   1750/2045  8786/8117
+    //   24 gadgets of 2 to 6      110/111   163/163   446/442   1465/1464  6194/6215
+    // (a second-order Trotter step of 21 qubits 343/279; a line at one and a
+    // half times the gates whatever r costs the last of these 552 at 24 and
+    // 1816 at 26 qubits.  No span passes at all cost layers with random gadgets
+    // 8190 us instead of 6620 at 25 qubits.)  force: the front gadget fits no
+    // tile, so a span pass takes it alone if need be
     auto spanFirst = [&](const OpView& left, size_t num, size_t tileGates, bool force) {
         const int ks = std::min(g_cfg.spanQubits, n - 1);
         if (ks < 10) return (size_t)0;
         const size_t r = spanRun(left, num, n, ks, std::min(low, ks - RB), span, spanProg);
-        return ((force && r >= 1) || (r >= 2 && 2 * r > 3 * tileGates)) ? r : (size_t)0;
+        return ((force && r >= 1) || (r >= 2 && 100 * r > tileGates * std::max<size_t>(100, 40 + 7 * r))) ? r : (size_t)0;
     };
     if (g_cfg.exact) {
         size_t i = 0;

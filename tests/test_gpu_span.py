@@ -125,15 +125,30 @@ def test_span_passes_in_default_mode(api):
         assert np.allclose(off, want, rtol=0, atol=1e-11), np.max(np.abs(off - want))
 
 
-@pytest.mark.parametrize("gadgets,passes", [(3, 0), (4, 1)])
-def test_span_pass_only_beyond_one_and_a_half_times_the_tile_pass(api, gadgets, passes):
+@pytest.mark.parametrize("gadgets,passes", [(2, 0), (3, 1), (4, 1)])
+def test_span_pass_of_few_gadgets_costs_a_tile_pass(api, gadgets, passes):
     """A tile of 12 qubits takes the first two gadgets, a span pass all of
-    them: three do not pay for it, four do.  Bitwise equal either way."""
+    them: one more pays for it.  Bitwise equal either way."""
     c = qc.Circuit(16, False, [], ("random", 21), f"line_{gadgets}")
     for k, (pauli, first) in enumerate([("XYXY", 4), ("YXXZ", 8), ("XXYX", 12), ("XYZX", 12)][:gadgets]):
         c.ops.append(("PG", pauli, list(range(first, first + 4)), 0.3 + 0.1 * k))
     c.ops.append(("U1", 4, qc.haar_unitary(qc.SplitMix64(5), 2)))
     say(f"span line case: {gadgets} gadgets")
+    want, _ = run(api, c, fused=False)
+    got, st = run(api, c, fused=True, shape=(12, 3, 2048))
+    assert st["passes"] == passes
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("last,passes", [(9, 0), (19, 0)])
+def test_span_pass_of_many_gadgets_costs_more(api, last, passes):
+    """Gadgets on neighbours: a span pass would take a few more than a tile
+    pass (16 to 10 of the longer line), and cost half as much again."""
+    c = qc.Circuit(20, False, [], ("random", 22), f"neighbours_{last}")
+    for k in range(last - 1):
+        for pauli in ("XZX", "YZY"):
+            c.ops.append(("PG", pauli, [k, k + 1, k + 2], 0.2 + 0.01 * k))
+    say(f"span cost case: neighbours up to {last}")
     want, _ = run(api, c, fused=False)
     got, st = run(api, c, fused=True, shape=(12, 3, 2048))
     assert st["passes"] == passes
