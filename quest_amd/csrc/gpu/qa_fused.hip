@@ -717,12 +717,15 @@ uint64_t supportMask(const GOp& g) {
 // the single-gate kernels; false, with v untouched, for a kind whose action is
 // not known on the host (a DENSEN matrix is in device memory).  The vectors are
 // unit vectors that some gates have been applied to, mostly zeros: pairs and
-// products of zeros are left out.
+// products of zeros are left out, as are those with a factor's zero part (a
+// gadget's are real and imaginary).
 template <typename R>
 bool applySmall(const GOp& g, const int* q, int nq, std::complex<R>* v) {
     typedef std::complex<R> cx;
     const cx zero(0);
     auto mul = [](const cx& x, const cx& y) {
+        if (x.imag() == 0) return cx(x.real() * y.real(), x.real() * y.imag());
+        if (x.real() == 0) return cx(-x.imag() * y.imag(), x.imag() * y.real());
         return cx(x.real() * y.real() - x.imag() * y.imag(), x.real() * y.imag() + x.imag() * y.real());
     };
     auto loc = [&](uint64_t m) {
@@ -968,9 +971,11 @@ void fuse::mergePass(const GOp* ops, size_t num, uint64_t localMask, std::vector
         std::vector<uint32_t> members;  // positions in ops, ascending
         bool dense;                     // some member is not diagonal
         bool matrix = false;            // some member is a matrix, or a Pauli tensor or gadget
+        bool gadget = false;            // some member is a Pauli tensor or gadget
         bool channel = false;           // some member is a damping or Pauli channel
         void note(const GOp& g) {
             matrix |= g.kind == F_DENSE1 || g.kind == F_DENSE2 || g.kind == F_PAULI;
+            gadget |= g.kind == F_PAULI;
             channel |= g.kind == F_DAMP1 || g.kind == F_PAULIS1;
         }
     };
@@ -992,7 +997,7 @@ void fuse::mergePass(const GOp* ops, size_t num, uint64_t localMask, std::vector
             if ((b.variants >> x) & 1ull) q[nq++] = x;
         const int D = 1 << nq, DL = 1 << nl;
         std::complex<double> M[64];
-        if (prec == QA_FP64) productOf<long double>(ops, b.members, q, nq, M);
+        if (prec == QA_FP64 && b.gadget) productOf<long double>(ops, b.members, q, nq, M);
         else productOf<double>(ops, b.members, q, nq, M);
         GOp g;
         g.t1 = q[0];
@@ -1049,6 +1054,7 @@ void fuse::mergePass(const GOp* ops, size_t num, uint64_t localMask, std::vector
                 nb.members.insert(nb.members.end(), open[b].members.begin(), open[b].members.end());
                 nb.dense |= open[b].dense;
                 nb.matrix |= open[b].matrix;
+                nb.gadget |= open[b].gadget;
                 nb.channel |= open[b].channel;
             } else {
                 emit(open[b]);

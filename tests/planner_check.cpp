@@ -816,8 +816,8 @@ static int blocksMain(int cases, uint64_t seed0) {
 
 // ---- merged matrices ----------------------------------------------------------
 
-// runs of gates on two qubits: the one matrix that they become is their product,
-// each element rounded once
+// runs of gates on two qubits, gadgets among them: the one matrix that they
+// become is their product, each element rounded once
 static int roundingMain(int cases, uint64_t seed0) {
     typedef std::complex<long double> lx;
     double worst = 0;
@@ -862,8 +862,10 @@ static int roundingMain(int cases, uint64_t seed0) {
             queue.push_back(g);
         }
         mergePass(queue.data(), queue.size(), (1ull << n) - 1ull, merged);
+        bool gadget = false;
+        for (const GOp& g : queue) gadget = gadget || g.kind == F_PAULI;
         bool dense = merged.size() == 1 && merged[0].kind == F_DENSE2;
-        if (!dense) {  // gates on one of the qubits only
+        if (!dense || !gadget) {
             if (merged.size() > 2) return std::printf("case %d: %zu ops\n", c, merged.size()), 1;
             continue;
         }
