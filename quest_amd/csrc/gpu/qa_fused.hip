@@ -964,7 +964,7 @@ void productOf(const GOp* ops, const std::vector<uint32_t>& members, const int* 
 
 }  // namespace fuse
 
-void fuse::mergePass(const GOp* ops, size_t num, uint64_t localMask, std::vector<GOp>& out, int prec) {
+void fuse::mergePass(const GOp* ops, size_t num, uint64_t localMask, std::vector<GOp>& out, bool extended) {
     struct Block {
         uint64_t qubits;                // local qubits
         uint64_t variants;              // non-local qubits (members are diagonal in them)
@@ -997,7 +997,7 @@ void fuse::mergePass(const GOp* ops, size_t num, uint64_t localMask, std::vector
             if ((b.variants >> x) & 1ull) q[nq++] = x;
         const int D = 1 << nq, DL = 1 << nl;
         std::complex<double> M[64];
-        if (prec == QA_FP64 && b.gadget) productOf<long double>(ops, b.members, q, nq, M);
+        if (extended && b.gadget) productOf<long double>(ops, b.members, q, nq, M);
         else productOf<double>(ops, b.members, q, nq, M);
         GOp g;
         g.t1 = q[0];
@@ -1813,7 +1813,8 @@ int flushQueue(void* amps, Queue& qu) {
         takePicked(ops.data(), left, picked, pass);
         const size_t numGates = pass.size();
         merged.clear();
-        mergePass(pass.data(), pass.size(), L, merged, qu.prec);
+        mergePass(pass.data(), pass.size(), L, merged,
+                  qu.prec == QA_FP64 && std::min(g_cfg.spanQubits, n - 1) >= 10);
         pass.clear();
         clusterPass(merged.data(), merged.size(), (1ull << low) - 1ull, pass);
         rc = launchPass(amps, qu, pass, 0, pass.size(), L, numGates);

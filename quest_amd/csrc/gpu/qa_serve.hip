@@ -467,7 +467,7 @@ bool launchStep(Engine& E, StepBuf& sb, std::string& err) {
                 layerPass(pass.data(), pass.size(), (1ull << low) - 1ull, merged);
                 pass.swap(merged);
             } else {
-                mergePass(pass.data(), pass.size(), L, merged, E.prec);
+                mergePass(pass.data(), pass.size(), L, merged);
                 pass.clear();
                 clusterPass(merged.data(), merged.size(), (1ull << low) - 1ull, pass);
             }

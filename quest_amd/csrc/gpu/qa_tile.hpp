@@ -72,13 +72,14 @@ void takePicked(const GOp* ops, std::vector<uint32_t>& left, const std::vector<u
 // (as controls or diagonal factors, which makes the run block-diagonal in
 // them) becomes one DENSE1V op: a 2x2 matrix per value of those qubits,
 // picked per tile.  Runs of diagonal gates only, and runs of one gate, are
-// emitted unchanged.  In a complex128 state, runs that hold gadgets are
-// multiplied in extended precision, which rounds each element once: where
-// Trotter steps repeat a matrix they repeat its rounding (21 qubits, XX, YY and
-// ZZ on pairs: error 1.27e-15, 1.42e-15 with products in FP64, 1.32e-15 where
-// most gadgets were in span passes), at 10 us of host time a step.  Others are
-// multiplied in FP64: 15 ns less a product, 3% of a 6-qubit noise study.
-void mergePass(const GOp* ops, size_t num, uint64_t localMask, std::vector<GOp>& out, int prec = QA_FP64);
+// emitted unchanged.  With `extended`, runs that hold gadgets are multiplied in
+// extended precision, which rounds each element once: where Trotter steps
+// repeat a matrix they repeat its rounding (21 qubits, XX, YY and ZZ on pairs:
+// error 1.27e-15, 1.42e-15 with products in FP64, 1.32e-15 where most gadgets
+// are in span passes).  It takes 0.1 us more a gadget, which a flush spends on
+// complex128 states that span passes reach (from 11 qubits; at 8 a Trotter
+// circuit of 76 us would take 85).
+void mergePass(const GOp* ops, size_t num, uint64_t localMask, std::vector<GOp>& out, bool extended = false);
 
 // the ops of one pass reordered so that ops on the same register group are
 // applied together: rounds that each take, in order, every op that commutes

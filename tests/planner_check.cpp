@@ -861,7 +861,7 @@ static int roundingMain(int cases, uint64_t seed0) {
             want = next;
             queue.push_back(g);
         }
-        mergePass(queue.data(), queue.size(), (1ull << n) - 1ull, merged);
+        mergePass(queue.data(), queue.size(), (1ull << n) - 1ull, merged, true);
         bool gadget = false;
         for (const GOp& g : queue) gadget = gadget || g.kind == F_PAULI;
         bool dense = merged.size() == 1 && merged[0].kind == F_DENSE2;

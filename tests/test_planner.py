@@ -51,9 +51,9 @@ def test_span_passes_act_like_the_gadgets(planner_check, seed):
 
 
 def test_merged_matrices_are_rounded_once(planner_check):
-    """The matrix of a run of gates on two qubits of a complex128 state, with
-    gadgets among them, is their product with each element rounded to FP64
-    once."""
+    """The matrix of a run of gates on two qubits, with gadgets among them, is
+    their product with each element rounded to FP64 once where a flush asks
+    for extended precision."""
     out = subprocess.run([str(planner_check), "300", "1", "rounding"], capture_output=True, text=True, timeout=120)
     assert out.returncode == 0, out.stdout + out.stderr
     assert "300 cases agree" in out.stdout
